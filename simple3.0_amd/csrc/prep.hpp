@@ -477,11 +477,12 @@ __device__ inline float prep_selec_wave(int k, int n, float* arr, int* ls, int* 
   }
 }
 
-// cosedge_1 (simple_math.f90:1089-1103) and cosedge_inner_1 (:1128-1140), FP32.
+// cosedge_1 (simple_math.f90:1089-1103) and cosedge_inner_1 (:1128-1140), FP32.  sqrtf is the correctly
+// rounded root, which decides the comparisons with the radii; __fsqrt_rn is the bare hardware root.
 __device__ __forceinline__ float prep_cosedge(float x, float y, int box, float mskrad) {
   const float pi32 = 3.14159274101257324f;
   const float maxrad = (float)(box / 2);
-  const float rad = __fsqrt_rn(x * x + y * y);
+  const float rad = sqrtf(x * x + y * y);
   const float width = 2.0f * (maxrad - mskrad);
   if (rad >= maxrad) return 0.0f;
   if (rad >= maxrad - width) return (cosf(((rad - (maxrad - width)) / width) * pi32) + 1.0f) / 2.0f;
@@ -489,7 +490,7 @@ __device__ __forceinline__ float prep_cosedge(float x, float y, int box, float m
 }
 __device__ __forceinline__ float prep_cosedge_inner(float x, float y, float width, float mskrad) {
   const float pi32 = 3.14159274101257324f;
-  const float rad = __fsqrt_rn(x * x + y * y);
+  const float rad = sqrtf(x * x + y * y);
   if (rad < mskrad - width) return 0.0f;
   if (rad > mskrad) return 1.0f;
   return (1.0f + cosf(pi32 * (mskrad - rad) / width)) / 2.0f;

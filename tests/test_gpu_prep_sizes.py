@@ -23,3 +23,22 @@ def test_prep_box_sizes(B, M):
     got = lib.prep_imgs(imgs, shifts, box=B, msk=msk)
     lib.kill()
     _check(got, imgs, shifts, P.PrepCfg(box=B, boxmatch=M, msk=msk), None)
+
+
+def test_inner_mask_starts_at_the_rounded_root():
+    """Pixels at distance sqrt(N) and an inner edge that starts at exactly that FP32 number: their weight
+    is 1 with the correctly rounded root, and about 1/2 with one that is an ulp too small (the edge is
+    two ulps wide)."""
+    B = 64
+    rng = np.random.default_rng(5)
+    imgs = _particles(rng, 1, B)
+    shifts = np.zeros((1, 2), np.float32)
+    lib = _handle(B)
+    roots = sorted({x * x + y * y for x in range(1, 20) for y in range(x + 1) if 16 < x * x + y * y < 400})
+    for N in roots[::3]:
+        inner = np.sqrt(np.float32(N))
+        width = np.float32(2) * np.spacing(inner)
+        say(f"inner mask radius sqrt({N})")
+        got = lib.prep_imgs(imgs, shifts, box=B, msk=24.0, inner=float(inner), width=float(width))
+        _check(got, imgs, shifts, P.PrepCfg(box=B, boxmatch=B, msk=24.0, inner=float(inner), width=float(width)), None)
+    lib.kill()

@@ -433,9 +433,13 @@ int pftcc_get_timing_channel(pftcc_t* h, int32_t channel, double* total_ms, int6
 
 /* Tile of the plain FP32 correlation kernel for an exhaustive search with ns shifts (0 =
  * unshifted): *tile = (reference, shift) pairs per work-group of the compile-time kernel (0: the
- * runtime-size kernel runs), *staged = 1 when the staged-reference variant runs; *tile is then the
- * fewest shifts with which it runs.  No reference counterpart (instrumentation). */
+ * runtime-size kernel runs), *staged = 1 when the staged-reference variant runs.  No reference
+ * counterpart (instrumentation). */
 int pftcc_get_corr_tile(const pftcc_t* h, int32_t ns, int32_t* tile, int32_t* staged);
+/* Fewest shifts with which the staged-reference variant runs for searches that have it (the CC
+ * objective without shell normalisation); 0: the runtime-size kernel runs.  No reference counterpart
+ * (instrumentation). */
+int pftcc_get_corr_min_shifts(const pftcc_t* h, int32_t* min_shifts);
 
 /* ------------------------------------------------------------------------- utilities -- */
 /* magic_pftsz (simple_magic_boxes.f90:25-37). */

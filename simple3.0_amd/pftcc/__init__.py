@@ -172,6 +172,7 @@ SIGNATURES = [
     ("pftcc_set_timing", _I, [_P, _I]),
     ("pftcc_get_timing", _I, [_P, _PD, C.POINTER(C.c_int64)]),
     ("pftcc_get_corr_tile", _I, [_P, _I, _PI, _PI]),
+    ("pftcc_get_corr_min_shifts", _I, [_P, _PI]),
     ("pftcc_magic_pftsz", _I, [_I]),
 ]
 
@@ -867,6 +868,12 @@ class PolarFTCorrCalc:
         st = C.c_int32()
         self._chk(self._lib.pftcc_get_corr_tile(self._h, int(nshifts), C.byref(t), C.byref(st)), "get_corr_tile")
         return t.value, bool(st.value)
+
+    def get_corr_min_shifts(self):
+        """Fewest shifts with which the staged-reference variant runs (0: runtime-size kernel)."""
+        m = C.c_int32()
+        self._chk(self._lib.pftcc_get_corr_min_shifts(self._h, C.byref(m)), "get_corr_min_shifts")
+        return m.value
 
     def set_stream(self, stream_ptr):
         self._chk(self._lib.pftcc_set_stream(self._h, C.c_void_p(stream_ptr)), "set_stream")

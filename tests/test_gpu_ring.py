@@ -53,8 +53,9 @@ def test_ring_kernels_equal_the_generic_kernel(n, monkeypatch):
         for ns in (0, 1, 5, 41):                # 41 shifts: the staged-reference variant (CC, no filter)
             say(f"ring kernels: n={n} {form} ns={ns}")
             tile, staged = lib.get_corr_tile(ns)
-            assert tile > 0 and bool(staged) == (ns >= 41 and not form.get("match_filt") and not form.get("euclid")) \
-                or ns == 5
+            plain = not form.get("match_filt") and not form.get("euclid")
+            assert tile > 0 and staged == (plain and ns >= lib.get_corr_min_shifts())
+            assert staged == plain or ns != 41
             got = lib.gencorrs_batch(ids, None, shift_list(ns))
             ref = gen.gencorrs_batch(ids, None, shift_list(ns))
             assert np.all(np.isfinite(got))

@@ -1,12 +1,11 @@
 """Parity of the staged-reference plain kernel (the exhaustive shift-grid search) with the oracle.
 
 The plain FP32 search switches to its staged-reference variant when a work-group's tile of
-(reference, shift) pairs spans at most two references, i.e. when the number of shifts is at least
-the tile: 9 at pftsz 308, 5 at 192 and 400, 32 at small sizes.  That variant stages the two
-references' |CTF|-weighted rows per shell in LDS, sums their FP64 norms from the staged rows, and
-orders work-groups tile-major over groups of 16 particles.  These tests run it (checked through
-pftcc_get_corr_tile) with tiles that straddle two references (nr x ns not a multiple of the tile)
-and particle counts that leave a partial group of 16, against:
+(reference, shift) pairs spans few references, i.e. from pftcc_get_corr_min_shifts shifts on.  That
+variant stages the spanned references' |CTF|-weighted rows per shell in LDS, sums their FP64 norms from
+the staged rows, and orders work-groups tile-major over groups of 16 particles.  These tests run it
+(checked through pftcc_get_corr_tile) with tiles that straddle references, a part-filled last tile
+(nr x ns not a multiple of the tile) and particle counts that leave a partial group of 16, against:
   * the FP64 oracle of gencorrs_cc_2 (simple_polarft_corrcalc.f90:1502-1534) for every vector:
     within 1e-5 of the peak, best rotation identical where the top-2 gap exceeds 10x the error;
   * the device's own full vectors for pftcc_search (first maximum in (ref, shift, rot) order);
@@ -37,11 +36,11 @@ def shift_grid(lim, step):
 
 
 @pytest.mark.parametrize("n,kto,ldim,shifts,nptcls,nrefs", [
-    (308, 60, 200, shift_grid(3.0, 0.5), 17, 3),     # 169 shifts, tile 9: 507 pairs, 3 left over
-    (192, 40, 128, shift_grid(1.5, 1.5)[:7], 21, 3),  # 7 shifts, tile 5
-    (400, 80, 256, shift_grid(1.0, 1.0), 17, 2),      # 9 shifts, tile 4
-    (500, 40, 320, shift_grid(1.0, 1.0), 17, 2),      # 9 shifts, tile 4
-    (16, 7, 32, shift_grid(2.0, 0.5)[:33], 18, 2),    # 33 shifts, tile 32
+    (308, 60, 200, shift_grid(3.0, 0.5), 17, 3),     # 169 shifts, 507 pairs
+    (192, 40, 128, shift_grid(1.5, 1.5)[:7], 21, 3),  # 7 shifts, 21 pairs
+    (400, 80, 256, shift_grid(1.0, 1.0), 17, 2),      # 9 shifts, 18 pairs
+    (500, 40, 320, shift_grid(1.0, 1.0), 17, 2),      # 9 shifts, 18 pairs
+    (16, 7, 32, shift_grid(2.0, 0.5)[:33], 18, 2),    # 33 shifts, 66 pairs
 ])
 def test_staged_reference_kernel_matches_oracle(n, kto, ldim, shifts, nptcls, nrefs):
     ns = len(shifts)
@@ -51,7 +50,10 @@ def test_staged_reference_kernel_matches_oracle(n, kto, ldim, shifts, nptcls, nr
     lib = to_lib(pf, cps)
     tile, staged = lib.get_corr_tile(ns)
     assert staged, (tile, ns)
-    assert (nrefs * ns) % tile != 0 and tile <= ns
+    assert ns >= lib.get_corr_min_shifts()
+    assert (nrefs * ns) % tile != 0                            # a part-filled last tile
+    assert any(f // ns != min(f + tile, nrefs * ns) // ns for f in range(0, nrefs * ns, tile)
+               if min(f + tile, nrefs * ns) % ns)              # a tile that straddles two references
     ids = np.arange(1, nptcls + 1)
     full = lib.gencorrs_batch(ids, None, shifts)               # [np][nr][ns][nrots]
     worst = 0.0
@@ -94,7 +96,7 @@ def test_staged_kernel_on_2d_classification_slice():
     refs_sel = np.sort(np.concatenate([src, others])).astype(np.int32)
     nr = len(refs_sel)
     tile, staged = lib.get_corr_tile(len(shifts))
-    assert staged and tile == 9
+    assert staged and (nr * len(shifts)) % tile != 0
     ids = np.arange(1, w.nptcls + 1)
     gcc, gir, gish, grot = lib.search(ids, refs_sel, shifts)
     refs = np.stack([lib.get_ref_pft(int(r), True) for r in refs_sel])

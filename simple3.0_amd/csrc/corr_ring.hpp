@@ -47,17 +47,35 @@ __device__ __forceinline__ float ldf(const float* __restrict__ base, unsigned in
   return *reinterpret_cast<const float*>(reinterpret_cast<const char*>(base) + (elem << 2));
 }
 
-// acc += conj(Z) w1 + Zn w2: the split and the product conj(V) W of one bin with the split's
-// m-dependent factors folded into w1 = conj(A') W and w2 = conj(B') W.
+// Ring lengths that had compile-time kernels before the table of lengths (ring_table.hpp).  Results
+// recorded with them stay as they are: their sums (ring_apart), their callback's order of operations
+// (rings.hip) and their FP16 spectra in the FP8 coarse pass (mfma_group).
+constexpr bool ring_first(int n) {
+  for (int m : {16, 24, 32, 40, 48, 64, 100, 192, 240, 308, 400, 500, 600})
+    if (n == m) return true;
+  return false;
+}
+
+// Whether a shell's product is formed on its own and then added to the sum over the shells, as the
+// runtime-size kernel does, instead of by multiply-adds onto the sum: one rounding of the sum per shell
+// and component instead of four, for two additions per bin.  Relative error of 5760 correlation vectors
+// against FP64: n 220 3.5e-7 -> 2.3e-7 (runtime-size kernel 2.5e-7), n 450 4.9e-7 -> 2.8e-7 (3.0e-7); the first
+// lengths' kernels always added onto the sum (n 400 4.5e-7).  200 particles x 50 references x 25 shifts
+// at n 220: 2.81 -> 2.92 ms; 150 x 500 at n 364: 4.04 -> 4.02 ms.
+constexpr bool ring_apart(int n) { return !ring_first(n); }
+
+// conj(Z) w1 + Zn w2, the split and the product conj(V) W of one bin with the split's m-dependent
+// factors folded into w1 = conj(A') W and w2 = conj(B') W: onto acc (APART: formed apart and added).
+template <bool APART>
 __device__ __forceinline__ void acc_w12(float2& acc, float2 Z, float2 Zn, float4 w) {
-  acc.x = fmaf(Z.x, w.x, acc.x);
-  acc.x = fmaf(Z.y, w.y, acc.x);
-  acc.y = fmaf(Z.x, w.y, acc.y);
-  acc.y = fmaf(-Z.y, w.x, acc.y);
-  acc.x = fmaf(Zn.x, w.z, acc.x);
-  acc.x = fmaf(-Zn.y, w.w, acc.x);
-  acc.y = fmaf(Zn.x, w.w, acc.y);
-  acc.y = fmaf(Zn.y, w.z, acc.y);
+  float2 p = APART ? make_float2(Z.x * w.x, Z.x * w.y) : make_float2(fmaf(Z.x, w.x, acc.x), fmaf(Z.x, w.y, acc.y));
+  p.x = fmaf(Z.y, w.y, p.x);
+  p.y = fmaf(-Z.y, w.x, p.y);
+  p.x = fmaf(Zn.x, w.z, p.x);
+  p.x = fmaf(-Zn.y, w.w, p.x);
+  p.y = fmaf(Zn.x, w.w, p.y);
+  p.y = fmaf(Zn.y, w.z, p.y);
+  acc = APART ? cadd(acc, p) : p;
 }
 
 // Y[m] of the inverse real FFT from X[m] and X[N-m]; e = exp(+i pi m / N).  Returns conj(Y).
@@ -117,20 +135,21 @@ __device__ __forceinline__ float lane_swap(float v) {
 __device__ __forceinline__ float2 lane_swap(float2 v) { return make_float2(lane_swap(v.x), lane_swap(v.y)); }
 
 // acc_w12 with Zn the neighbouring lane's Zm, read by the multiply-adds themselves (a quad permutation
-// of their first operand) instead of by two moves: 80 of 977 instructions of a shell at n 400.  The leading wait covers the hazard between the
-// instruction that wrote Zm and the first that permutes it.
+// of their first operand) instead of by two moves: 80 of 977 instructions of a shell at n 400.  The
+// leading wait covers the hazard between the instruction that wrote Zm and the first that permutes it.
+template <bool APART>
 __device__ __forceinline__ void acc_w12_swap(float2& acc, float2 Z, float2 Zm, float4 w) {
-  acc.x = fmaf(Z.x, w.x, acc.x);
-  acc.x = fmaf(Z.y, w.y, acc.x);
-  acc.y = fmaf(Z.x, w.y, acc.y);
-  acc.y = fmaf(-Z.y, w.x, acc.y);
+  float2 p = APART ? make_float2(Z.x * w.x, Z.x * w.y) : make_float2(fmaf(Z.x, w.x, acc.x), fmaf(Z.x, w.y, acc.y));
+  p.x = fmaf(Z.y, w.y, p.x);
+  p.y = fmaf(-Z.y, w.x, p.y);
   asm("s_nop 1\n\t"
       "v_fmac_f32_dpp %0, %2, %4 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
       "v_fmac_f32_dpp %1, %2, %5 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
       "v_fmac_f32_dpp %0, -%3, %5 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
       "v_fmac_f32_dpp %1, %3, %4 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf"
-      : "+v"(acc.x), "+v"(acc.y)
+      : "+v"(p.x), "+v"(p.y)
       : "v"(Zm.x), "v"(Zm.y), "v"(w.z), "v"(w.w));
+  acc = APART ? cadd(acc, p) : p;
 }
 
 // Row k1 (0 .. A, row A being row 0 with its outputs shifted by one) of one transform (buf at the
@@ -253,7 +272,7 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(W))) k_
   constexpr int T1 = F * B, TPT1 = (T1 + NT - 1) / NT;
   constexpr int TF = RP == 2 ? R::G : 2 * R::G;     // last-pass tasks per transform
   constexpr int TL = F * TF, TPTL = (TL + NT - 1) / NT;
-  constexpr bool PFA = ring_pfa<N, A, RST>();
+  constexpr bool PFA = ring_pfa<N, A, RST>(), APART = ring_apart(N);
   constexpr int WL = ring_wlen<N, A, RST>(), RR = RST ? ring_rows(N, F, RP) : 1;
   constexpr int WS = PFA ? A + 1 : A;        // stride of a row's staged bins
   extern __shared__ __align__(16) float2 smem[];
@@ -529,13 +548,13 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(W))) k_
           const float4* wb = Wk4 + A - row;
           static_for<0, B>([&](auto tt) {
             constexpr int T = decltype(tt)::value, TM = PFA ? (B - T) % B : B - 1 - T;
-            acc_w12(acc[c][T], y1[T], y2[TM], wa[WS * T]);
-            acc_w12(acc[c][B + T], y2[T], y1[TM], wb[WS * T]);
+            acc_w12<APART>(acc[c][T], y1[T], y2[TM], wa[WS * T]);
+            acc_w12<APART>(acc[c][B + T], y2[T], y1[TM], wb[WS * T]);
           });
         } else {
           static_for<0, B>([&](auto tt) {
             constexpr int T = decltype(tt)::value, TM = PFA ? (B - T) % B : B - 1 - T;
-            acc_w12_swap(acc[c][T], y1[T], y1[TM], wa[WS * T]);
+            acc_w12_swap<APART>(acc[c][T], y1[T], y1[TM], wa[WS * T]);
           });
         }
       }

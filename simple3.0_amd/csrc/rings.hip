@@ -62,13 +62,8 @@ struct Ring {
   }
   // shift-search items: shells per work-group pass (LDS for four work-groups per CU), and threads
   static constexpr int IF = N <= 400 ? 8 : 4, IT = N <= 64 ? 64 : 256;
-  // lengths whose items have a compile-time kernel; the others' order of operations is the runtime-size
-  // kernel's
-  static constexpr bool has_items() {
-    for (int m : {16, 24, 32, 40, 48, 64, 100, 192, 240, 308, 400, 500, 600})
-      if (N == m) return true;
-    return false;
-  }
+  // the other lengths' callback keeps the runtime-size kernel's order of operations
+  static constexpr bool has_items() { return ring_first(N); }
   static void items(hipStream_t s, const CorrArgs& a) {
     if constexpr (has_items())
       hipLaunchKernelGGL((k_corr_items<N, IF, IT>), dim3((unsigned)a.np), dim3(IT),

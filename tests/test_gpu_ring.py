@@ -164,3 +164,31 @@ def test_shift_search_callback_equals_the_generic_kernel(n, monkeypatch):
         assert np.max(np.abs(cxy[:, 1:] - ref[:, 1:])) < 1e-2
         lib.kill()
         gen.kill()
+
+
+@pytest.mark.parametrize("n", [132, 176, 220, 364, 450, 546])
+@pytest.mark.parametrize("ns", [0, 25])
+def test_ring_kernel_keeps_the_generic_kernel_s_accuracy(n, ns, monkeypatch):
+    """Lengths whose searches ran on the runtime-size kernel: the relative error of whole vectors against
+    FP64, over searches large enough that no shells are split, is not larger than that kernel's.  0.15
+    covers the scatter of the two estimates (48 pairs and more, each over 2 n rotations)."""
+    nptcls, nrefs = 480, 3 if ns else 12
+    say(f"accuracy of the ring kernel: n={n} ns={ns}")
+    pf, cps = make_case(seed=n + ns, n=n, kfrom=2, kto=n // 5, ctf=True, astig=0.3, nrefs=nrefs, nptcls=nptcls,
+                        ldim=2 * (n // 3))
+    for i in range(nptcls):
+        pf.ptcls[i] = (pf.refs_even[i % nrefs] + pf.ptcls[i]).astype(np.complex64)
+    sh = shift_list(ns)
+    err = []
+    for h in both(monkeypatch, pf, cps):
+        got = h.gencorrs_batch(np.arange(1, nptcls + 1), None, sh).reshape(nptcls, nrefs, max(ns, 1), -1)
+        h.kill()
+        num = den = 0.0
+        for i in range(0, nptcls, 120 if ns else 60):
+            for r in range(min(nrefs, 6)):
+                exact = pf.gencorrs_shifts(r, i, sh) if ns else [pf.gencorrs(r, i, None, method="fft")]
+                num += np.sum((got[i, r] - np.stack(exact)) ** 2)
+                den += np.sum(np.square(exact))
+        err.append(np.sqrt(num / den))
+    say(f"  relative error {err[0]:.2e}, runtime-size kernel {err[1]:.2e}")
+    assert err[0] < 1.15 * err[1]

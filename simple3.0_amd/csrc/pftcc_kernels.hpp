@@ -504,12 +504,7 @@ struct Rot8Args {
   int npairs;
   double* f;                   // [npairs]
   double* grad;                // [npairs][3] or null
-  // shells split over work-groups: chunk c takes kper shells and leaves its kRot8Sums sums in
-  // part [npairs][nsplit][kRot8Sums], k_rot8_finish adds them in chunk order (nsplit 1: not split)
-  int nsplit, kper;
-  double* part;
 };
-constexpr int kRot8Sums = 6;   // objective, d/dx, d/dy, d/dpsi numerators, reference and particle norms
 
 // One block of 256 threads per (ref, particle, shift, rotation) item; threads own angles j and
 // run the shells in order so the shift phase follows gen_shmat_8's recurrence (:1098-1120).
@@ -587,9 +582,11 @@ __device__ __forceinline__ void rot8_step(const Rot8Args a, const Rot8Shell& s, 
 }
 
 // Shells of loads in flight ahead of the arithmetic in k_rot8, and wavefronts per SIMD its registers must
-// allow.  Many items hide their latency by wavefronts (9000 pairs at n 308, 69 shells: 0.53 ms with 1
+// allow.  Many items hide their latency by wavefronts (9000 pairs at n 308, 69 shells: 0.52 ms with 1
 // ahead at 7 wavefronts, 0.62 with 4 ahead at 4); few items by loads ahead (shift search of 1000
-// pairs: 10.5 ms with 1 ahead, 10.1 with 4, 10.3 with 6 to 12).
+// pairs: 10.5 ms with 1 ahead, 10.1 with 4, 10.3 with 6 to 12).  Both take an item's sums in the same order,
+// whatever the items beside it: spreading the shells of a few items over work-groups took one item at
+// n 192 from 16 to 7 us, but a line search that is driven item by item or in batches then saw other bits.
 constexpr int kRot8Ahead = 1, kRot8Waves = 7;
 constexpr int kRot8AheadFew = 4, kRot8WavesFew = 1;
 
@@ -603,30 +600,6 @@ __global__ void __launch_bounds__(256) k_shell_sq8(const float2* __restrict__ ri
   for (int j = threadIdx.x & 63; j < n; j += 64) s += (double)v[j].x * v[j].x + (double)v[j].y * v[j].y;
   for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
   if ((threadIdx.x & 63) == 0) out[it] = s;
-}
-
-// f and the gradient of one item from its sums.
-__device__ __forceinline__ void rot8_result(const Rot8Args& a, int item, int mode, const double (&v)[kRot8Sums]) {
-  double den = 1.0;
-  if (mode == 1) den = sqrt(v[4] * (double)a.sqsums[a.ips[item]]);
-  else if (mode == 0) den = sqrt(v[4] * v[5]);
-  a.f[item] = v[0] / den;
-  if (a.grad) {
-    a.grad[3 * (size_t)item] = v[1] / den;
-    a.grad[3 * (size_t)item + 1] = v[2] / den;
-    a.grad[3 * (size_t)item + 2] = mode == 2 ? 0.0 : v[3] / den;
-  }
-}
-
-__global__ void k_rot8_finish(Rot8Args a) {
-  const int item = blockIdx.x * blockDim.x + threadIdx.x;
-  if (item >= a.npairs) return;
-  double v[kRot8Sums] = {0, 0, 0, 0, 0, 0};
-  const double* p = a.part + (size_t)item * a.nsplit * kRot8Sums;
-  for (int c = 0; c < a.nsplit; ++c)
-#pragma unroll
-    for (int u = 0; u < kRot8Sums; ++u) v[u] += p[c * kRot8Sums + u];
-  rot8_result(a, item, a.mode, v);
 }
 
 // Threads own angles j and run the shells in order.  The loads of shell k + D are issued before
@@ -650,19 +623,19 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(W))) k
   const float* ctf = a.ctf ? a.ctf + (size_t)ip * a.nk * n : nullptr;
   const bool angle = dpt != nullptr;
   Rot8Acc acc;
-  const int kb = a.nsplit > 1 ? blockIdx.y * a.kper : 0;
-  const int ke = a.nsplit > 1 ? min(a.kcorr, kb + a.kper) : a.kcorr;
+  // the first shell, a number that the compiler does not know: with a literal 0 it keeps an address per
+  // array and shell of the unrolled loop, and spills more (9000 pairs at n 308: 579 us, so 519)
+  int kb = 0;
+  asm("" : "+s"(kb));
   // k-weighted particle norm from the per-shell FP64 sums, one shell per thread
-  if (MODE == 0 && blockIdx.y == 0)
+  if (MODE == 0)
     for (int kk = threadIdx.x; kk < a.kcorr; kk += blockDim.x)
       acc.sqptcl += (double)(a.kfrom + kk) * a.sqp8[(size_t)ip * a.nk + kk];
   for (int j = threadIdx.x; j < n; j += blockDim.x) {
     const float snj = a.sn32[j], ncnj = a.ncn32[j];
     double sa, ca, ss, cs;
-    // phase of shell kb: the first shell's, kb steps on (the recurrence's product in closed form)
-    const double step = a.one_x[j] * sx + a.one_y[j] * sy;
-    sincos(a.argx[j] * sx + a.argy[j] * sy + (double)kb * step, &sa, &ca);
-    sincos(step, &ss, &cs);
+    sincos(a.argx[j] * sx + a.argy[j] * sy, &sa, &ca);
+    sincos(a.one_x[j] * sx + a.one_y[j] * sy, &ss, &cs);
     double shr = ca, shi = sa;
     int t = j + rho;           // index of P on the full ring (mod 2n)
     bool cj = false;
@@ -670,22 +643,23 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(W))) k
     if (t >= n) { t -= n; cj = true; }
     // a ring of D + 1 shells: shell m lives in slot m % (D + 1); the loads of shell m + D are
     // issued before the arithmetic of shell m
+    const int kc = a.kcorr;
     Rot8Shell s[D + 1];
 #pragma unroll
     for (int u = 0; u < D; ++u)
-      if (kb + u < ke) rot8_load<MODE, NORM>(a, s[u], kb + u, j, t, ip, iref, even, ref, ptc, dpt, ctf);
+      if (kb + u < kc) rot8_load<MODE, NORM>(a, s[u], kb + u, j, t, ip, iref, even, ref, ptc, dpt, ctf);
     int kk = kb;
-    for (; kk + D + 1 <= ke; kk += D + 1) {
+    for (; kk + D + 1 <= kc; kk += D + 1) {
 #pragma unroll
       for (int u = 0; u <= D; ++u) {
-        if (kk + u + D < ke) rot8_load<MODE, NORM>(a, s[(u + D) % (D + 1)], kk + u + D, j, t, ip, iref, even, ref, ptc, dpt, ctf);
+        if (kk + u + D < kc) rot8_load<MODE, NORM>(a, s[(u + D) % (D + 1)], kk + u + D, j, t, ip, iref, even, ref, ptc, dpt, ctf);
         rot8_step<MODE, NORM>(a, s[u], kk + u, cj, angle, snj, ncnj, acc, shr, shi, cs, ss);
       }
     }
 #pragma unroll
     for (int u = 0; u <= D; ++u)
-      if (kk + u < ke) {
-        if (kk + u + D < ke) rot8_load<MODE, NORM>(a, s[(u + D) % (D + 1)], kk + u + D, j, t, ip, iref, even, ref, ptc, dpt, ctf);
+      if (kk + u < kc) {
+        if (kk + u + D < kc) rot8_load<MODE, NORM>(a, s[(u + D) % (D + 1)], kk + u + D, j, t, ip, iref, even, ref, ptc, dpt, ctf);
         rot8_step<MODE, NORM>(a, s[u], kk + u, cj, angle, snj, ncnj, acc, shr, shi, cs, ss);
       }
   }
@@ -702,15 +676,18 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(W))) k
   __syncthreads();
   if (threadIdx.x == 0) {
     const int nw = (blockDim.x + 63) >> 6;
-    double v[kRot8Sums];
-    for (int u = 0; u < kRot8Sums; ++u) {
+    // objective, d/dx, d/dy, d/dpsi numerators, reference and particle norms
+    double v[6];
+    for (int u = 0; u < 6; ++u) {
       v[u] = red[u][0];
       for (int w = 1; w < nw; ++w) v[u] += red[u][w];
     }
-    if (a.nsplit > 1) {
-      for (int u = 0; u < kRot8Sums; ++u) a.part[((size_t)item * a.nsplit + blockIdx.y) * kRot8Sums + u] = v[u];
-    } else {
-      rot8_result(a, item, MODE, v);
+    const double den = MODE == 2 ? 1.0 : sqrt(v[4] * (MODE == 1 ? (double)a.sqsums[ip] : v[5]));
+    a.f[item] = v[0] / den;
+    if (a.grad) {
+      a.grad[3 * (size_t)item] = v[1] / den;
+      a.grad[3 * (size_t)item + 1] = v[2] / den;
+      a.grad[3 * (size_t)item + 2] = MODE == 2 ? 0.0 : v[3] / den;
     }
   }
 }

@@ -192,3 +192,24 @@ def test_ring_kernel_keeps_the_generic_kernel_s_accuracy(n, ns, monkeypatch):
         err.append(np.sqrt(num / den))
     say(f"  relative error {err[0]:.2e}, runtime-size kernel {err[1]:.2e}")
     assert err[0] < 1.15 * err[1]
+
+
+@pytest.mark.parametrize("form", [dict(), dict(match_filt=True), dict(euclid=True)])
+def test_objective_of_an_item_is_the_same_in_every_batch(form):
+    """The FP64 objective and gradient of an item have the same bits alone, among a few and among many
+    (the batches of 1024 and 1025 items lie on both sides of k_rot8's variants)."""
+    say(f"objective in batches: {form}")
+    pf, cps = make_case(seed=29, n=192, kfrom=2, kto=40, ctf=True, nrefs=3, nptcls=8, ldim=128, eo_mixed=True, **form)
+    lib = to_lib(pf, cps)
+    rng = np.random.default_rng(4)
+    n = 1025
+    r, p, o = rng.integers(1, 4, n), rng.integers(1, 9, n), rng.integers(1, 385, n)
+    sh = rng.uniform(-4, 4, (n, 2))
+    f, g = lib.grad_batch(r, p, sh, o)
+    for k in (1, 3, 40, 1024):
+        fk, gk = lib.grad_batch(r[:k], p[:k], sh[:k], o[:k])
+        assert np.array_equal(fk, f[:k]) and np.array_equal(gk, g[:k]), k
+    for i in range(5):
+        f1, g1 = lib.gencorr_grad_for_rot_8(r[i], p[i], sh[i], o[i])
+        assert f1 == f[i] and np.array_equal(g1, g[i, :2])
+    lib.kill()

@@ -225,7 +225,10 @@ int pftcc_calc_roinv_corrmat(pftcc_t* h, float* corrmat);
  * iptcls[np] (global ids), irefs[nr] (1-based; NULL = all refs 1..nr), shifts[ns][2]
  * (NULL with ns == 0 selects the unshifted gencorrs_1 semantics).
  * cc_out layout: [np][nr][max(ns,1)][nrots] (host memory).  This is what a loop of
- * gencorrs(iref, iptcl[, shvec], cc) over the same lists returns, bit-compatible with it. */
+ * gencorrs(iref, iptcl[, shvec], cc) over the same lists returns, bit-compatible with it where fewer
+ * than pftcc_get_corr_min_shifts shifts are given (from there on the staged-reference variant runs, and
+ * the two agree within FP32 rounding).  A pair's vector does not depend on the other particles and
+ * references of the call, here and in every search below. */
 int pftcc_gencorrs_batch(pftcc_t* h, int32_t np, const int32_t* iptcls, int32_t nr,
                          const int32_t* irefs, int32_t ns, const float* shifts, float* cc_out);
 /* The same search reduced on the device: for each particle the best (ref, shift, irot) over

@@ -78,6 +78,21 @@ __device__ __forceinline__ void acc_w12(float2& acc, float2 Z, float2 Zn, float4
   acc = APART ? cadd(acc, p) : p;
 }
 
+// (w1, w2) of acc_w12 at a bin with spectrum value w, shell weight wk and t = exp(-i pi m / N).
+__device__ __forceinline__ float4 spec_w12(float2 w, float wk, float2 t) {
+  const float2 wh = make_float2(wk * w.x, wk * w.y);
+  const float2 w1 = cmul(make_float2(1.f + t.y, t.x), wh), w2 = cmul(make_float2(1.f - t.y, -t.x), wh);
+  return make_float4(w1.x, w1.y, w2.x, w2.y);
+}
+
+// Particle's share of the normalisation: the sum of squares, or (Euclid) of the weighted shells'.
+__device__ __forceinline__ float ring_pscal(const CorrArgs& a, int ip) {
+  if (a.mode != 1) return a.sqsums[ip];
+  float s = 0.f;
+  for (int kk = 0; kk < a.kcorr; ++kk) s += a.shellw[(size_t)ip * a.nk + kk] * a.sqsums_k[(size_t)ip * a.nk + kk];
+  return s;
+}
+
 // Y[m] of the inverse real FFT from X[m] and X[N-m]; e = exp(+i pi m / N).  Returns conj(Y).
 __device__ __forceinline__ float2 unsplit_bin_conj(float2 X, float2 Xn, float2 e) {
   const float2 s = make_float2(X.x + Xn.x, X.y - Xn.y);
@@ -175,6 +190,54 @@ __device__ __forceinline__ int ring_row(int r) {
   return RP == 2 ? r : (r & 1) ? A - (r >> 1) : (r >> 1);
 }
 
+// Output of one pair's transform: normalised values to cc_out, the best (cc, first position) into key.
+struct RingEmit {
+  float scale, off;
+  int n;
+  __device__ __forceinline__ RingEmit(const CorrArgs& a, int n, float sq, float o, float ps) : off(o + ps), n(n) {
+    const float inv4n = 1.0f / (4.0f * (float)n);
+    scale = a.mode == 1 ? inv4n : inv4n / sqrtf(sq * ps);
+  }
+  // output m of particle slot pi's pair P: rotations 2 m and 2 m + 1
+  __device__ __forceinline__ void operator()(const CorrArgs& a, int pi, int npairs, int P, int m, float2 y,
+                                             unsigned long long& key) const {
+    float x0 = y.x, x1 = -y.y;
+    if (a.mode == 1) {
+      x0 = 2.f * x0 * scale - off;
+      x1 = 2.f * x1 * scale - off;
+    } else {
+      x0 *= scale;
+      x1 *= scale;
+    }
+    if (a.cc_out) reinterpret_cast<float2*>(a.cc_out + ((size_t)pi * npairs + P) * (2 * n))[m] = make_float2(x0, x1);
+    if (a.best) {
+      const unsigned int lin0 = (unsigned int)P * (unsigned int)(2 * n) + 2u * m;
+      const unsigned long long k0 = ((unsigned long long)ordered_bits(x0) << 32) | (0xFFFFFFFFu - lin0);
+      const unsigned long long k1 = ((unsigned long long)ordered_bits(x1) << 32) | (0xFFFFFFFFu - lin0 - 1u);
+      key = k0 > key ? k0 : key;
+      key = k1 > key ? k1 : key;
+    }
+  }
+};
+
+// The work-group's best key into *best: wavefront maxima, then the wavefronts' in a fixed order.
+template <int NT>
+__device__ __forceinline__ void ring_best(unsigned long long* best, unsigned long long key, unsigned long long* red,
+                                          int tid) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    const unsigned long long v = __shfl_xor(key, o);
+    key = v > key ? v : key;
+  }
+  if ((tid & 63) == 0) red[tid >> 6] = key;
+  __syncthreads();
+  if (tid == 0) {
+    unsigned long long m = red[0];
+    for (int w = 1; w < NT / 64; ++w) m = red[w] > m ? red[w] : m;
+    atomicMax(best, m);
+  }
+}
+
 // Inverse real transform of F accumulated spectra held as acc[slot][RP B] by the tasks of the last
 // pass: emit(f, m, y) gets output m, rotations 2m (y.x) and
 // 2m + 1 (-y.y).  buf is free; every thread of the work-group calls it.
@@ -232,13 +295,15 @@ __device__ __forceinline__ void ring_inverse(const float2 (&acc)[TPTL][RP * (N /
   }
 }
 
-// Partial sums of a search whose shells are split over work-groups: spectra zpart [pair][chunk][N+1]
-// and npart [pair][chunk] = (sum |q|^2, Euclid offset), pair = particle slot x (nr ns) + P.
+// A search whose shells are split over work-groups: they leave every shell's transform, zrow
+// [pair][kcorr][B][A + 1] (row A as in ring_last_row), and (per-pair variant) its slots' sums |q|^2,
+// es [pair][shells][B]; k_ring_finish multiplies and sums them in the order of the unsplit kernel, so a
+// pair's result does not depend on the launch.  pair = particle slot x (nr ns) + P.
 struct RingSplit {
   int nsplit;                  // shell chunks (1: not split)
   int kper;                    // shells per chunk
-  float2* zpart;
-  double2* npart;
+  float2* zrow;
+  float* es;
 };
 
 // The staged-reference kernel takes the Good-Thomas form where it can: its operands (staged rows,
@@ -265,7 +330,8 @@ constexpr size_t ring_lds_bytes(int rows) {
 // references: the shell's CTF-weighted reference rows are staged once per work-group in LDS and each
 // reference's norm is summed from them (|ref x CTF x shmat|^2 = |ref x CTF|^2), instead of per pair.
 // PRF: pass 1 loads its global operand (per-pair: reference values, RST: shift phases) a shell ahead.
-template <int N, int A, int F, int NT, int W, int RP, bool RST, bool PRF>
+// SPLIT: only the transforms, of the shells of one chunk (RingSplit).
+template <int N, int A, int F, int NT, int W, int RP, bool RST, bool PRF, bool SPLIT>
 __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(W))) k_corr_ring(CorrArgs a, RingSplit sp) {
   using R = RingGeom<N, A>;
   constexpr int B = R::B, H = R::H, S = R::S;
@@ -300,7 +366,6 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(W))) k_
   const int rem = t - grp * GRP * a.ntiles;
   const int tile = rem / gsz;
   const int pi = grp * GRP + (rem - tile * gsz);
-  const int chunk = blockIdx.y;
   const int ip = a.plist[pi];
   const bool even = a.iseven[ip] != 0;
   const float2* refs = even ? a.refs_even : a.refs_odd;
@@ -311,8 +376,8 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(W))) k_
   const int live = min(F, npairs - tile * F), t1 = live * B, tl = live * TF;
   const bool EUC = !RST && a.mode == 1;
   const int kloop = a.kcorr > a.knorm ? a.kcorr : a.knorm;
-  const int kb = sp.nsplit > 1 ? chunk * sp.kper : 0;
-  const int ke = sp.nsplit > 1 ? min(kloop, kb + sp.kper) : kloop;
+  const int kb = SPLIT ? (int)blockIdx.y * sp.kper : 0;
+  const int ke = SPLIT ? min(kloop, kb + sp.kper) : kloop;
 
   if constexpr (!PFA) ring_twiddles<N, A, NT>(tw, a.tw2g, tid);
 
@@ -393,7 +458,7 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(W))) k_
     }
   };
   auto fetch_spec = [&](int k) {
-    if (k < a.kcorr)
+    if (!SPLIT && k < a.kcorr)
 #pragma unroll
       for (int u = 0; u < MP; ++u) {
         const int m = tid + u * NT;
@@ -415,7 +480,7 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(W))) k_
             if (r < nrow) {
               const float2 q = make_float2(prr[r][u].x * cv, prr[r][u].y * cv);
               rck[r * N + jp] = make_float2(q.x, __uint_as_float(__float_as_uint(q.y) ^ sgn));
-              rsum[r] += (double)(q.x * q.x + q.y * q.y);
+              rsum[r] += (double)fmaf(q.y, q.y, q.x * q.x);
             }
         } else {
           ctfk[j] = pcv[u];
@@ -441,15 +506,11 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(W))) k_
     const bool docorr = kk < a.kcorr;
     const bool donorm = RST || kk < a.knorm;
     const float wk = (EUC && docorr) ? a.shellw[(size_t)ip * nk + kk] : 1.0f;
-    if (docorr)
+    if (!SPLIT && docorr)
 #pragma unroll
       for (int u = 0; u < MP; ++u) {
         const int m = tid + u * NT;
-        if (m <= N) {
-          const float2 wh = make_float2(wk * pwm[u].x, wk * pwm[u].y), tm = twm[u];
-          const float2 w1 = cmul(make_float2(1.f + tm.y, tm.x), wh), w2 = cmul(make_float2(1.f - tm.y, -tm.x), wh);
-          Wk4[PFA ? R::pfa_wpos(m) : m] = make_float4(w1.x, w1.y, w2.x, w2.y);
-        }
+        if (m <= N) Wk4[PFA ? R::pfa_wpos(m) : m] = spec_w12(pwm[u], wk, twm[u]);
       }
     if (kk + 1 < ke) {
       fetch_rows(kk + 1);
@@ -522,6 +583,7 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(W))) k_
         });
       }
       if constexpr (!RST) {
+        if constexpr (SPLIT) sp.es[(((size_t)pi * npairs + tile * F + f) * kloop + kk) * B + t3] = e2;
         if (donorm) sqp[c] += e2;
         if (EUC && docorr) offp[c] = fmaf(wk, e2, offp[c]);
       }
@@ -542,7 +604,11 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(W))) k_
         float2 y1[B];
         ring_last_row<N, A, PFA>(buf + f * S, tw, row, y1);
         const float4* wa = Wk4 + row;
-        if constexpr (RP == 2) {
+        if constexpr (SPLIT) {
+          static_assert(RP == 1, "a row per task");
+          float2* z = sp.zrow + (((size_t)pi * npairs + tile * F + f) * a.kcorr + kk) * (B * (A + 1)) + row;
+          static_for<0, B>([&](auto tt) { z[decltype(tt)::value * (A + 1)] = y1[decltype(tt)::value]; });
+        } else if constexpr (RP == 2) {
           float2 y2[B];
           ring_last_row<N, A, PFA>(buf + f * S, tw, A - row, y2);
           const float4* wb = Wk4 + A - row;
@@ -560,6 +626,7 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(W))) k_
       }
     __syncthreads();
   }
+  if constexpr (SPLIT) return;
   // ---- normalisation sums (fixed order) ----
   float* sqs = reinterpret_cast<float*>(Wk4);
   float* offs = sqs + T1;
@@ -594,159 +661,130 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(W))) k_
     }
     sq[f] = (float)s0;
     off[f] = (float)s1;
-    const int P = tile * F + f;
-    if (sp.nsplit > 1 && P < npairs)
-      sp.npart[((size_t)pi * npairs + P) * sp.nsplit + chunk] = make_double2(s0, s1);
   }
-  if (sp.nsplit > 1) {
-    // this chunk's spectra; k_ring_finish sums the chunks and transforms
-#pragma unroll
-    for (int c = 0; c < TPTL; ++c) {
-      const int task = tid + c * NT;
-      const int f = task / TF, row = ring_row<A, RP>(task % TF);
-      const int P = tile * F + f;
-      if (task >= TL || P >= npairs) continue;
-      float2* z = sp.zpart + (((size_t)pi * npairs + P) * sp.nsplit + chunk) * (N + 1);
-      // row A (the mirror of row 0) holds the Nyquist bin: PFA output 0, else output B - 1
-      auto put = [&](int rw, auto tt, float2 v) {
-        constexpr int T = decltype(tt)::value;
-        if (rw != A) z[PFA ? R::pfa_bin(rw, T) : rw + A * T] = v;
-        else if (T == (PFA ? 0 : B - 1)) z[N] = v;
-      };
-      static_for<0, B>([&](auto tt) {
-        put(row, tt, acc[c][decltype(tt)::value]);
-        if constexpr (RP == 2) put(A - row, tt, acc[c][B + decltype(tt)::value]);
-      });
-    }
-    return;
-  }
-  if (tid == 0) {
-    if (a.mode == 1) {
-      float s = 0.f;
-      for (int kk = 0; kk < a.kcorr; ++kk) s += a.shellw[(size_t)ip * nk + kk] * a.sqsums_k[(size_t)ip * nk + kk];
-      pscal = s;
-    } else {
-      pscal = a.sqsums[ip];
-    }
-  }
+  if (tid == 0) pscal = ring_pscal(a, ip);
   if constexpr (PFA) ring_twiddles<N, A, NT>(tw, a.tw2g, tid);   // the spectra are no longer read
   // ---- inverse transform of every pair, normalisation, output ----
-  const float inv4n = 1.0f / (4.0f * (float)N);
   unsigned long long bestkey = 0ull;
   ring_inverse<N, A, F, NT, RP, TPTL, PFA>(acc, buf, tw, a.tw2g, tid, [&](int f, int m, float2 y) {
     const int P = tile * F + f;
-    if (P >= npairs) return;
-    float x0 = y.x, x1 = -y.y;
-    if (a.mode == 1) {
-      const float o = off[f] + pscal;
-      x0 = 2.f * x0 * inv4n - o;
-      x1 = 2.f * x1 * inv4n - o;
-    } else {
-      const float sc = inv4n / sqrtf(sq[f] * pscal);
-      x0 *= sc;
-      x1 *= sc;
-    }
-    if (a.cc_out) {
-      float2* o = reinterpret_cast<float2*>(a.cc_out + ((size_t)pi * npairs + P) * (2 * N));
-      o[m] = make_float2(x0, x1);
-    }
-    if (a.best) {
-      const unsigned int lin0 = (unsigned int)P * (unsigned int)(2 * N) + 2u * m;
-      const unsigned long long k0 = ((unsigned long long)ordered_bits(x0) << 32) | (0xFFFFFFFFu - lin0);
-      const unsigned long long k1 = ((unsigned long long)ordered_bits(x1) << 32) | (0xFFFFFFFFu - lin0 - 1u);
-      bestkey = k0 > bestkey ? k0 : bestkey;
-      bestkey = k1 > bestkey ? k1 : bestkey;
-    }
+    if (P < npairs) RingEmit(a, N, sq[f], off[f], pscal)(a, pi, npairs, P, m, y, bestkey);
   });
-  if (a.best) {
-    // wavefront maxima, then the wavefronts' in a fixed order
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-      const unsigned long long v = __shfl_xor(bestkey, o);
-      bestkey = v > bestkey ? v : bestkey;
-    }
-    if ((tid & 63) == 0) red[tid >> 6] = bestkey;
-    __syncthreads();
-    if (tid == 0) {
-      unsigned long long m = red[0];
-      for (int w = 1; w < NT / 64; ++w) m = red[w] > m ? red[w] : m;
-      atomicMax(&a.best[pi], m);
-    }
-  }
+  if (a.best) ring_best<NT>(a.best + pi, bestkey, red, tid);
 }
 
 // Finishes a search whose shells were split over work-groups: the work-group of a pair (particle slot x
-// npairs + P) sums its chunks' spectra in chunk order and their norms, then runs the inverse
-// transform, the normalisation and the output of k_corr_ring.
-// Bound: the latency of the chunks' loads, so a thread owns MB bins and keeps 8 chunks of each in
-// flight, and the norms are loaded a chunk per lane.  160 pairs x 47 chunks at n 240: 70 -> 8 us against
-// four pairs per work-group whose threads walked the chunks one by one.
-template <int N, int A, int NT>
+// npairs + P) runs the products, sums, inverse transform, normalisation and output of k_corr_ring on the
+// transforms left in sp, in the same order of operations (row A's bins, the mirror of row 0, have
+// sums of their own there and here).  RST: the reference's norm is summed from its rows, as there.
+// Bound: the latency of the loads, so a thread owns MB bins and keeps UB shells of each in flight.  Call of
+// 160 pairs x 47 shells at n 240: 57 us, as with the chunks' sums added by 160 work-groups; 152 us
+// unsplit through the kernels before.
+template <int N, int A, bool RST, int NT>
 __global__ void __launch_bounds__(NT) k_ring_finish(CorrArgs a, RingSplit sp, int npairs) {
   using R = RingGeom<N, A>;
-  constexpr int B = R::B, S = R::S, MB = (N + NT) / NT, UB = 8;
+  constexpr int B = R::B, S = R::S, A1 = A + 1, ZL = A1 * B, MB = (ZL + NT - 1) / NT, UB = 16 / MB;
+  constexpr bool PFA = ring_pfa<N, A, RST>(), APART = ring_apart(N);
   static_assert(A <= NT && B <= NT && NT % 64 == 0, "one task per thread");
   extern __shared__ __align__(16) float2 smem[];
   float2* buf = smem;                        // [S]
   float2* tw = buf + S;
-  float2* Z = tw + R::TW;                    // [N + 1]
-  __shared__ float norm[3];                  // sum |q|^2, Euclid offset, particle scale
+  float2* Z = tw + R::TW;                    // [ZL]
+  __shared__ float sqs[B], offs[B], norm[3]; // norm: sum |q|^2, Euclid offset, particle scale
+  __shared__ double rsq[NT / 64];
   __shared__ unsigned long long red[NT / 64];
   const int tid = threadIdx.x, lane = tid & 63;
-  const int pair = blockIdx.x, pi = pair / npairs;
+  const int pair = blockIdx.x, pi = pair / npairs, P = pair - pi * npairs;
+  const int ip = a.plist[pi], nk = a.nk, kc = a.kcorr, kloop = kc > a.knorm ? kc : a.knorm;
   ring_twiddles<N, A, NT>(tw, a.tw2g, tid);
-  if (tid < 64) {
-    double s0 = 0.0, s1 = 0.0;
-    for (int c = lane; c < sp.nsplit; c += 64) {
-      const double2 v = sp.npart[(size_t)pair * sp.nsplit + c];
-      s0 += v.x;
-      s1 += v.y;
-    }
-    const int ip = a.plist[pi];
-    float ps = 0.f;
-    if (a.mode == 1) {
-      for (int kk = lane; kk < a.kcorr; kk += 64)
-        ps = fmaf(a.shellw[(size_t)ip * a.nk + kk], a.sqsums_k[(size_t)ip * a.nk + kk], ps);
-    } else if (lane == 0) {
-      ps = a.sqsums[ip];
-    }
+  if constexpr (RST) {
+    constexpr int JP = (N + NT - 1) / NT;
+    const int ir = P / a.ns, iref = a.rlist ? a.rlist[ir] : ir;
+    const float2* ref = (a.iseven[ip] ? a.refs_even : a.refs_odd) + (size_t)iref * nk * N;
+    const float* ctf = a.ctf ? a.ctf + (size_t)ip * nk * N : nullptr;
+    double s = 0.0;
+#pragma unroll 8
+    for (int kk = 0; kk < kloop; ++kk)
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-      s0 += __shfl_xor(s0, o);
-      s1 += __shfl_xor(s1, o);
-      ps += __shfl_xor(ps, o);
+      for (int u = 0; u < JP; ++u) {
+        const int j = tid + u * NT;
+        if (N % NT == 0 || j < N) {
+          const float cv = ctf ? ctf[kk * N + j] : 1.0f;
+          const float2 r = ref[kk * N + j], q = make_float2(r.x * cv, r.y * cv);
+          s += (double)fmaf(q.y, q.y, q.x * q.x);
+        }
+      }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
+    if (lane == 0) rsq[tid >> 6] = s;
+  } else if (tid < B) {
+    const float* e = sp.es + (size_t)pair * kloop * B + tid;
+    float s = 0.f, o = 0.f;
+#pragma unroll 8
+    for (int kk = 0; kk < kloop; ++kk) {
+      const float e2 = e[kk * B];
+      if (kk < a.knorm) s += e2;
+      if (a.mode == 1 && kk < kc) o = fmaf(a.shellw[(size_t)ip * nk + kk], e2, o);
     }
-    if (lane == 0) {
-      norm[0] = (float)s0;
-      norm[1] = (float)s1;
-      norm[2] = ps;
-    }
+    sqs[tid] = s;
+    offs[tid] = o;
   }
+  if (tid == NT - 1) norm[2] = ring_pscal(a, ip);
   {
-    const float2* z = sp.zpart + (size_t)pair * sp.nsplit * (N + 1);
-    float2 acc[MB];
+    const float2* z = sp.zrow + (size_t)pair * kc * ZL;
+    const float2* memo = a.memo + (size_t)ip * nk * (N + 1);
+    int iz[MB], in[MB], im[MB];
+    float2 acc[MB], tm[MB];
 #pragma unroll
-    for (int b = 0; b < MB; ++b) acc[b] = make_float2(0.f, 0.f);
-    for (int u0 = 0; u0 < sp.nsplit; u0 += UB) {
-      float2 v[UB][MB];
+    for (int b = 0; b < MB; ++b) {
+      const int i = min(tid + b * NT, ZL - 1), T = i / A1, row = i - T * A1;
+      iz[b] = i;
+      in[b] = (PFA ? (B - T) % B : B - 1 - T) * A1 + A - row;
+      im[b] = row == A ? (PFA ? N : A * (T + 1)) : PFA ? R::pfa_bin(row, T) : row + A * T;
+      acc[b] = make_float2(0.f, 0.f);
+      tm[b] = a.tw2g[im[b]];
+    }
+    for (int k0 = 0; k0 < kc; k0 += UB) {
+      float2 v[UB][MB], vn[UB][MB], w[UB][MB];
 #pragma unroll
       for (int u = 0; u < UB; ++u)
 #pragma unroll
-        for (int b = 0; b < MB; ++b)
-          v[u][b] = z[(size_t)min(u0 + u, sp.nsplit - 1) * (N + 1) + min(tid + b * NT, N)];
+        for (int b = 0; b < MB; ++b) {
+          const int k = min(k0 + u, kc - 1);
+          v[u][b] = z[k * ZL + iz[b]];
+          vn[u][b] = z[k * ZL + in[b]];
+          w[u][b] = memo[k * (N + 1) + im[b]];
+        }
 #pragma unroll
       for (int u = 0; u < UB; ++u)
-        if (u0 + u < sp.nsplit)
+        if (k0 + u < kc) {
+          const float wk = a.mode == 1 ? a.shellw[(size_t)ip * nk + k0 + u] : 1.0f;
 #pragma unroll
-          for (int b = 0; b < MB; ++b) acc[b] = cadd(acc[b], v[u][b]);
+          for (int b = 0; b < MB; ++b) acc_w12<APART>(acc[b], v[u][b], vn[u][b], spec_w12(w[u][b], wk, tm[b]));
+        }
     }
 #pragma unroll
     for (int b = 0; b < MB; ++b)
-      if (tid + b * NT <= N) Z[tid + b * NT] = acc[b];
+      if (tid + b * NT < ZL) Z[tid + b * NT] = acc[b];
   }
   __syncthreads();
-  for (int m = tid; m < N; m += NT) {
-    float2 X = Z[m], Xn = Z[N - m];
+  if (tid == 0) {
+    double s0 = 0.0, s1 = 0.0;
+    if constexpr (RST) {
+      for (int w = 0; w < NT / 64; ++w) s0 += rsq[w];
+    } else {
+      for (int u = 0; u < B; ++u) {
+        s0 += sqs[u];
+        s1 += offs[u];
+      }
+    }
+    norm[0] = (float)s0;
+    norm[1] = (float)s1;
+  }
+  for (int i = tid; i < N; i += NT) {
+    const int T = i / A, row = i - T * A, TM = PFA ? (B - T) % B : B - 1 - T;
+    const int m = PFA ? R::pfa_bin(row, T) : row + A * T;
+    float2 X = Z[T * A1 + row], Xn = Z[TM * A1 + (PFA && row == 0 && T != 0 ? 0 : A - row)];
     if (m == 0) {
       X.y = 0.f;
       Xn.y = 0.f;
@@ -764,44 +802,14 @@ __global__ void __launch_bounds__(NT) k_ring_finish(CorrArgs a, RingSplit sp, in
   __syncthreads();
   unsigned long long bestkey = 0ull;
   if (tid < A) {
-    const float inv4n = 1.0f / (4.0f * (float)N), sc = inv4n / sqrtf(norm[0] * norm[2]), o = norm[1] + norm[2];
-    float2* cc = a.cc_out ? reinterpret_cast<float2*>(a.cc_out + (size_t)pair * (2 * N)) : nullptr;
-    const unsigned int lin = (unsigned int)(pair % npairs) * (unsigned int)(2 * N);
     float2 y[B];
     ring_last_row<N, A, false>(buf, tw, tid, y);
+    const RingEmit e(a, N, norm[0], norm[1], norm[2]);
     static_for<0, B>([&](auto t) {
-      constexpr int T = decltype(t)::value;
-      const int m = tid + A * T;
-      float x0 = y[T].x, x1 = -y[T].y;
-      if (a.mode == 1) {
-        x0 = 2.f * x0 * inv4n - o;
-        x1 = 2.f * x1 * inv4n - o;
-      } else {
-        x0 *= sc;
-        x1 *= sc;
-      }
-      if (cc) cc[m] = make_float2(x0, x1);
-      const unsigned int lin0 = lin + 2u * m;
-      const unsigned long long k0 = ((unsigned long long)ordered_bits(x0) << 32) | (0xFFFFFFFFu - lin0);
-      const unsigned long long k1 = ((unsigned long long)ordered_bits(x1) << 32) | (0xFFFFFFFFu - lin0 - 1u);
-      const unsigned long long k = k0 > k1 ? k0 : k1;
-      bestkey = k > bestkey ? k : bestkey;
+      e(a, pi, npairs, P, tid + A * decltype(t)::value, y[decltype(t)::value], bestkey);
     });
   }
-  if (a.best) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-      const unsigned long long v = __shfl_xor(bestkey, o);
-      bestkey = v > bestkey ? v : bestkey;
-    }
-    if (lane == 0) red[tid >> 6] = bestkey;
-    __syncthreads();
-    if (tid == 0) {
-      unsigned long long m = red[0];
-      for (int w = 1; w < NT / 64; ++w) m = red[w] > m ? red[w] : m;
-      atomicMax(&a.best[pi], m);
-    }
-  }
+  if (a.best) ring_best<NT>(a.best + pi, bestkey, red, tid);
 }
 
 // Ring spectra (memoize_ffts :848-877): dst[i][kk][m] = rfft_2n(Re p + Im p | Re p - Im p)[m] of ring

@@ -12,10 +12,13 @@ struct RingOps {
   int tile, tile_rst;          // pairs per work-group of the plain search (per-pair / staged references)
   int min_shifts;              // fewest shifts with which the staged-reference variant runs
   int pfa_a;                   // its radix A where it takes the Good-Thomas form (shift table in that order), else 0
+  // a split search's memory per pair: values per shell of its transform (per-pair / staged variant), and
+  // the per-pair variant's sums |q|^2 per shell
+  int zrow, zrow_rst, slots;
   // plain search: grid (particle slots x tiles, shell chunks)
   void (*corr)(bool rst, dim3 grid, hipStream_t s, const pfk::CorrArgs& a, const pfk::RingSplit& sp);
   // finishes a search split over shell chunks: total pairs, npairs per particle slot
-  void (*finish)(int total, int npairs, hipStream_t s, const pfk::CorrArgs& a, const pfk::RingSplit& sp);
+  void (*finish)(bool rst, int total, int npairs, hipStream_t s, const pfk::CorrArgs& a, const pfk::RingSplit& sp);
   // shift-search items (a.np items, a.shtab their phases), or null: the runtime-size kernel takes them
   void (*items)(hipStream_t s, const pfk::CorrArgs& a);
   // inverse stage of the precision form: cnt particles against nr operand rows (a.Z16: FP16 spectra)

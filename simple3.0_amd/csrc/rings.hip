@@ -48,17 +48,28 @@ struct Ring {
   static constexpr int NT = 256;
   static constexpr RingCfg P = ring_row_of(N).pair, S = ring_row_of(N).staged;
   static void corr(bool rst, dim3 grid, hipStream_t s, const CorrArgs& a, const RingSplit& sp) {
-    if (rst)
-      hipLaunchKernelGGL((k_corr_ring<N, S.A, S.F, NT, S.W, S.RP, true, S.PRF>), grid, dim3(NT),
-                         (ring_lds_bytes<N, S.A, S.F, NT, true>(ring_span(S.F, a.ns))), s, a, sp);
+    const size_t lds_r = ring_lds_bytes<N, S.A, S.F, NT, true>(ring_span(S.F, a.ns));
+    constexpr size_t lds = ring_lds_bytes<N, P.A, P.F, NT, false>(0);
+    if (rst && sp.nsplit > 1)
+      hipLaunchKernelGGL((k_corr_ring<N, S.A, S.F, NT, 2, 1, true, false, true>), grid, dim3(NT), lds_r, s, a, sp);
+    else if (rst)
+      hipLaunchKernelGGL((k_corr_ring<N, S.A, S.F, NT, S.W, S.RP, true, S.PRF, false>), grid, dim3(NT), lds_r, s, a, sp);
+    else if (sp.nsplit > 1)
+      hipLaunchKernelGGL((k_corr_ring<N, P.A, P.F, NT, 2, 1, false, false, true>), grid, dim3(NT), lds, s, a, sp);
     else
-      hipLaunchKernelGGL((k_corr_ring<N, P.A, P.F, NT, P.W, P.RP, false, P.PRF>), grid, dim3(NT),
-                         (ring_lds_bytes<N, P.A, P.F, NT, false>(0)), s, a, sp);
+      hipLaunchKernelGGL((k_corr_ring<N, P.A, P.F, NT, P.W, P.RP, false, P.PRF, false>), grid, dim3(NT), lds, s, a, sp);
   }
-  static void finish(int total, int npairs, hipStream_t s, const CorrArgs& a, const RingSplit& sp) {
-    using R = RingGeom<N, P.A>;
-    hipLaunchKernelGGL((k_ring_finish<N, P.A, NT>), dim3((unsigned)total), dim3(NT),
-                       8 * (size_t)(R::S + R::TW + N + 1), s, a, sp, npairs);
+  template <int A>
+  static constexpr int zrow() { return (A + 1) * (N / A); }
+  template <int A, bool RST>
+  static void finish_go(int total, int npairs, hipStream_t s, const CorrArgs& a, const RingSplit& sp) {
+    using R = RingGeom<N, A>;
+    hipLaunchKernelGGL((k_ring_finish<N, A, RST, NT>), dim3((unsigned)total), dim3(NT),
+                       8 * (size_t)(R::S + R::TW + zrow<A>()), s, a, sp, npairs);
+  }
+  static void finish(bool rst, int total, int npairs, hipStream_t s, const CorrArgs& a, const RingSplit& sp) {
+    if (rst) finish_go<S.A, true>(total, npairs, s, a, sp);
+    else finish_go<P.A, false>(total, npairs, s, a, sp);
   }
   // shift-search items: shells per work-group pass (LDS for four work-groups per CU), and threads
   static constexpr int IF = N <= 400 ? 8 : 4, IT = N <= 64 ? 64 : 256;
@@ -85,7 +96,8 @@ struct Ring {
     hipLaunchKernelGGL((k_ring_spec<N, P.A, XF, 128>), dim3((unsigned)(((size_t)count * nk + XF - 1) / XF)), dim3(128),
                        8 * (size_t)(XF * R::S + R::TW), s, src, list, count, nk, tw2g, dst);
   }
-  static constexpr RingOps ops{N, P.F, S.F, ring_min_shifts(N, S.F, S.RP), ring_pfa<N, S.A, true>() ? S.A : 0, corr, finish,
+  static constexpr RingOps ops{N, P.F, S.F, ring_min_shifts(N, S.F, S.RP), ring_pfa<N, S.A, true>() ? S.A : 0,
+                               zrow<P.A>(), zrow<S.A>(), N / P.A, corr, finish,
                                has_items() ? items : nullptr, zifft, spec};
 };
 

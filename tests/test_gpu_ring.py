@@ -213,3 +213,26 @@ def test_objective_of_an_item_is_the_same_in_every_batch(form):
         f1, g1 = lib.gencorr_grad_for_rot_8(r[i], p[i], sh[i], o[i])
         assert f1 == f[i] and np.array_equal(g1, g[i, :2])
     lib.kill()
+
+
+@pytest.mark.parametrize("n", LENGTHS)
+def test_pair_is_the_same_in_every_launch(n):
+    """A pair's vector has the same bits alone (its shells spread over work-groups, k_ring_finish), among a
+    few and among 400 particles x 3 references (not spread: more than half of 768 work-groups)."""
+    for form in FORMS:
+        kw = dict(ctf=True, kstop=11)
+        kw.update(form)
+        pf, cps = make_case(seed=2 * n, n=n, kfrom=2, kto=13, nrefs=3, nptcls=400, ldim=max(40, n), eo_mixed=True, **kw)
+        lib = to_lib(pf, cps)
+        ids = np.arange(1, 401)
+        for ns in (0, 1, 41):
+            say(f"one pair, few pairs, many pairs: n={n} {form} ns={ns}")
+            sh = shift_list(ns)
+            many = lib.gencorrs_batch(ids, None, sh).reshape(400, 3, max(ns, 1), -1)
+            few = lib.gencorrs_batch(ids[5:8], None, sh).reshape(3, 3, max(ns, 1), -1)
+            one = lib.gencorrs_batch(ids[9:10], np.array([2], np.int32), sh).reshape(max(ns, 1), -1)
+            assert np.array_equal(few, many[5:8]), (form, ns, np.mean(few != many[5:8]))
+            assert np.array_equal(one, many[9, 1]), (form, ns, np.mean(one != many[9, 1]))
+            if ns < 2:
+                assert np.array_equal(lib.gencorrs(3, 11, sh[0] if ns else None), many[10, 2, 0])
+        lib.kill()

@@ -114,3 +114,16 @@ def test_noalloc_search_limits_and_errors():
     ref = lib.search(np.arange(1, 5, dtype=np.int32), None, None)
     assert np.array_equal(ok[1], ref[1]) and np.array_equal(ok[3], ref[3])
     lib.kill()
+
+
+def test_searches_agree_whatever_memory_a_split_may_take():
+    """Few particles and many shifts: the shells are spread over work-groups where memory allows it, which
+    the static scratch does not beside this shift table.  The three forms give the same bits."""
+    say("host, device and no-alloc search: n 308, K 59, 4 particles x 2 references x 169 shifts")
+    pf, cps = make_case(seed=613, n=308, kfrom=2, kto=60, ctf=True, nrefs=2, nptcls=4, ldim=200)
+    lib = to_lib(pf, cps)
+    ids, sh = np.arange(1, 5, dtype=np.int32), shift_grid(3.0, 0.5)
+    host = lib.search(ids, None, sh)
+    for fn in (lib.search_dev, lib.search_dev_noalloc):
+        _same(_search(lib, fn, ids, None, sh, _outputs(4)), host)
+    lib.kill()

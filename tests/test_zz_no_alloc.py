@@ -127,3 +127,27 @@ def test_searches_agree_whatever_memory_a_split_may_take():
     for fn in (lib.search_dev, lib.search_dev_noalloc):
         _same(_search(lib, fn, ids, None, sh, _outputs(4)), host)
     lib.kill()
+
+
+def _held_by(fn):
+    """Device memory that a call leaves allocated."""
+    torch.cuda.synchronize()
+    free0 = torch.cuda.mem_get_info()[0]
+    fn()
+    torch.cuda.synchronize()
+    return free0 - torch.cuda.mem_get_info()[0]
+
+
+def test_fp16_spectra_take_four_bytes_per_value():
+    """FP8 coarse pass at n 100, 8000 references x 256 particles: FP16 spectra of 0.83 GB in one block."""
+    n, nr, npt = 100, 8000, 256
+    say(f"memory after an FP8 search: n {n}, {npt} particles x {nr} references")
+    pf, cps = make_case(seed=615, n=n, kfrom=2, kto=7, ctf=True, astig=0.0, nrefs=nr, nptcls=npt, ldim=64)
+    lib = to_lib(pf, cps)
+    ids = np.arange(1, npt + 1, dtype=np.int32)
+    lib.search_mfma(ids[:64], np.arange(1, 65, dtype=np.int32), prec=pftcc.PFTCC_PREC_FP8, ntop=4)
+    held = _held_by(lambda: lib.search_mfma(ids, None, prec=pftcc.PFTCC_PREC_FP8, ntop=4))
+    spectra, operand = (n + 1) * nr * npt * 4, (n + 1) * nr * 128
+    say(f"  held {held / 2 ** 20:.0f} MiB, spectra {spectra / 2 ** 20:.0f} MiB")
+    assert held < 1.2 * (spectra + operand)
+    lib.kill()

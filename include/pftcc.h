@@ -81,7 +81,8 @@ int pftcc_new(const pftcc_cfg* cfg, int32_t nrefs, int32_t pfrom, int32_t pto,
 /* kill (:2234-2279) */
 int pftcc_kill(pftcc_t* h);
 const char* pftcc_last_error(const pftcc_t* h);
-/* Asynchronous work is issued on this stream (hipStream_t; NULL = the null stream). */
+/* Asynchronous work is issued on this stream (hipStream_t; NULL = the null stream).  Work that earlier
+ * calls left in flight on another stream is waited for by this one: the handle's workspaces serve both. */
 int pftcc_set_stream(pftcc_t* h, void* hip_stream);
 int pftcc_sync(pftcc_t* h);
 

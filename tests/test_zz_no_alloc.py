@@ -167,3 +167,31 @@ def test_fp16_spectra_take_four_bytes_per_value():
     say(f"  held {held / 2 ** 20:.0f} MiB, spectra {spectra / 2 ** 20:.0f} MiB")
     assert held < 1.2 * (spectra + operand)
     lib.kill()
+
+
+def test_calls_on_another_stream_wait_for_work_in_flight():
+    """A search left in flight on one stream, then a shift search and a gradient on another: both use the
+    handle's workspaces, and the results are those of the calls one by one."""
+    say("two streams, one handle: n 308, 12 particles x 6 references")
+    pf, cps = make_case(seed=616, n=308, kfrom=2, kto=40, ctf=True, nrefs=6, nptcls=12, ldim=200)
+    for i in range(12):
+        pf.ptcls[i] = (pf.refs_even[i % 6] + 0.3 * pf.ptcls[i]).astype(np.complex64)
+    lib = to_lib(pf, cps)
+    ids = np.arange(1, 13, dtype=np.int32)
+    refs = (ids - 1) % 6 + 1
+    outs = _outputs(12)
+    alone = _search(lib, lib.search_dev, ids, None, None, outs)
+    cxy, rot = lib.shsrch_grad_batch(refs, ids, trs=3.0)
+    d_ids = _dev(ids, torch.int32)
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    torch.cuda.synchronize()
+    for _ in range(3):
+        lib.set_stream(streams[0].cuda_stream)
+        lib.search_dev(12, d_ids.data_ptr(), 6, None, 0, None, *(t.data_ptr() for t in outs))
+        lib.set_stream(streams[1].cuda_stream)
+        cxy2, rot2 = lib.shsrch_grad_batch(refs, ids, trs=3.0)
+        torch.cuda.synchronize()
+        _same(tuple(t.cpu().numpy() for t in outs), alone)
+        assert np.array_equal(cxy2, cxy) and np.array_equal(rot2, rot)
+    lib.set_stream(0)
+    lib.kill()

@@ -195,3 +195,32 @@ def test_calls_on_another_stream_wait_for_work_in_flight():
         assert np.array_equal(cxy2, cxy) and np.array_equal(rot2, rot)
     lib.set_stream(0)
     lib.kill()
+
+
+def test_handles_made_and_killed_by_several_threads():
+    """Pinned blocks go from handle to handle: six threads make, use and kill handles of their own."""
+    import threading
+    say("handles of six threads: n 48, 4 particles x 3 references")
+    cases = [make_case(seed=620 + t, n=48, kfrom=2, kto=14, ctf=True, nrefs=3, nptcls=4, ldim=64) for t in range(6)]
+    ids = np.arange(1, 5, dtype=np.int32)
+
+    def use(t):
+        lib = to_lib(*cases[t])
+        got = lib.gencorrs_batch(ids), lib.gencorrs(2, 3, (0.5, -1.0)), lib.search(ids)
+        lib.kill()
+        return got[0], got[1], *got[2]
+
+    want = [use(t) for t in range(6)]
+    wrong = []
+
+    def work(t):
+        for _ in range(8):
+            if not all(np.array_equal(a, b) for a, b in zip(use(t), want[t])):
+                wrong.append(t)
+
+    threads = [threading.Thread(target=work, args=(t,)) for t in range(6)]
+    for th in threads:
+        th.start()
+    for th in threads:
+        th.join()
+    assert not wrong, wrong

@@ -144,6 +144,9 @@ int pftcc_get_ptcl_pft(pftcc_t* h, int32_t iptcl, float* pft);                  
 int pftcc_get_ctfmat(pftcc_t* h, int32_t iptcl, float* ctfmat);
 int pftcc_get_memo(pftcc_t* h, int32_t iptcl, float* memo);
 int pftcc_get_sqsum_ptcl(pftcc_t* h, int32_t iptcl, float* sqsum);
+/* Ring spectra of the listed references (irefs[nr], 1-based) as the precision form takes them, for
+ * verification: out float[nr][nk][pftsz+1][2], laid out like a particle's memo. */
+int pftcc_get_ref_spectra(pftcc_t* h, int32_t nr, const int32_t* irefs, int32_t iseven, float* out);
 
 /* ------------------------------------------------------------------------- calculators -- */
 /* gencorrs (:173, 1594-1617): cc[nrots].  shvec == NULL selects gencorrs_1, else gencorrs_2

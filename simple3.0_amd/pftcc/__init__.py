@@ -124,6 +124,7 @@ SIGNATURES = [
     ("pftcc_get_ctfmat", _I, [_P, _I, _PF]),
     ("pftcc_get_memo", _I, [_P, _I, _PF]),
     ("pftcc_get_sqsum_ptcl", _I, [_P, _I, _PF]),
+    ("pftcc_get_ref_spectra", _I, [_P, _I, _PI, _I, _PF]),
     ("pftcc_gencorrs", _I, [_P, _I, _I, _PF, _PF]),
     ("pftcc_gencorr_for_rot", _I, [_P, _I, _I, _PF, _I, _PF]),
     ("pftcc_gencorr_for_rot_8", _I, [_P, _I, _I, _PD, _I, _PD]),
@@ -444,6 +445,14 @@ class PolarFTCorrCalc:
     def get_memo(self, iptcl):
         out = np.zeros((self.nk, self.pftsz + 1), np.complex64)
         self._chk(self._lib.pftcc_get_memo(self._h, iptcl, _fp(out.view(np.float32))), "get_memo")
+        return out
+
+    def get_ref_spectra(self, irefs, iseven=True):
+        """Ring spectra [nr, nk, n+1] of the listed references, as the precision form takes them."""
+        r = np.ascontiguousarray(irefs, np.int32)
+        out = np.zeros((r.size, self.nk, self.pftsz + 1), np.complex64)
+        self._chk(self._lib.pftcc_get_ref_spectra(self._h, r.size, _ip(r), int(iseven), _fp(out.view(np.float32))),
+                  "get_ref_spectra")
         return out
 
     def get_sqsum_ptcl(self, iptcl):

@@ -95,17 +95,27 @@ def test_split_search_equals_the_whole_one(n, ns):
 
 
 @pytest.mark.parametrize("n", LENGTHS)
-def test_ring_spectra_and_inverse_stage(n, monkeypatch):
-    """Ring spectra (k_ring_spec) against k_memoize; packing, contraction and inverse stage
-    (k_ring_zifft) of the precision form against the plain search, for ring-constant |CTF|.
-    Tolerance: the split-BF16 bar of 1e-4 of the peak and the plain search's 1e-5."""
+def test_ring_spectra_and_inverse_stage(n):
+    """Ring spectra of listed references (k_ring_spec, 8 rings per work-group) and of particles
+    (k_memoize) against FP64 transforms; packing, contraction and inverse stage (k_ring_zifft) of the
+    precision form against the plain search, for ring-constant |CTF|.
+    Tolerance: 1e-5 of a ring's peak; the split-BF16 bar of 1e-4 of the peak and the plain search's 1e-5."""
     say(f"ring spectra and inverse stage: n={n}")
     pf, cps = make_case(seed=7 * n, n=n, kfrom=2, kto=8, kstop=7, ctf=True, astig=0.0, nrefs=23, nptcls=9,
                         ldim=max(40, n), eo_mixed=True)
-    lib, gen = both(monkeypatch, pf, cps)
+    lib = to_lib(pf, cps)
+
+    def spectra(rings):                 # rfft_2n(Re p + Im p | Re p - Im p), memoize_ffts
+        p = rings.astype(np.complex128)
+        return np.fft.rfft(np.concatenate([p.real + p.imag, p.real - p.imag], axis=-1), axis=-1)
+
+    for iseven, refs in ((True, [23, 1, 7, 7, 2]), (False, [5]), (False, np.arange(1, 24))):
+        exact = spectra((pf.refs_even if iseven else pf.refs_odd)[np.array(refs) - 1]).reshape(-1, n + 1)
+        got = lib.get_ref_spectra(refs, iseven).reshape(-1, n + 1)
+        assert max(peak_rel_err(a, b) for a, b in zip(got, exact)) < FP32_TOL, (iseven, refs)
     for i in (1, 9):
-        assert peak_rel_err(lib.get_memo(i), gen.get_memo(i)) < 2 * FP32_TOL
-    gen.kill()
+        exact = spectra(pf.ptcls[i - 1])
+        assert max(peak_rel_err(a, b) for a, b in zip(lib.get_memo(i), exact)) < FP32_TOL
     ids = np.array([9, 2, 5, 1, 3])
     refs = np.concatenate([np.arange(23, 1, -2), np.arange(2, 23, 3)]).astype(np.int32)
     for ns in (0, 4):

@@ -18,6 +18,7 @@
 #include "lds_passes.hpp"
 #include "fft_lds.hpp"
 #include "pftcc_kernels.hpp"
+#include "selec.hpp"
 
 namespace pfk {
 
@@ -351,131 +352,15 @@ __global__ void __launch_bounds__(256) k_prep_rows_inv(const float2* __restrict_
   }
 }
 
-// selec (simple_math.f90:2204-2261), restated step for step on an LDS array (1-based indices as
-// the reference's; arr permuted in place).  Its final test compares ir - 1 with 1.
-__host__ __device__ float prep_selec(int k, int n, float* arr) {
-  int l = 1, ir = n;
-  auto A = [&](int i) -> float& { return arr[i - 1]; };
-  for (;;) {
-    if (ir - l <= 1) {
-      if (ir - 1 == 1 && A(ir) < A(l)) {
-        const float t = A(l);
-        A(l) = A(ir);
-        A(ir) = t;
-      }
-      return A(k);
-    }
-    const int mid = (l + ir) / 2;
-    float t = A(mid);
-    A(mid) = A(l + 1);
-    A(l + 1) = t;
-    if (A(l) > A(ir)) { t = A(l); A(l) = A(ir); A(ir) = t; }
-    if (A(l + 1) > A(ir)) { t = A(l + 1); A(l + 1) = A(ir); A(ir) = t; }
-    if (A(l) > A(l + 1)) { t = A(l); A(l) = A(l + 1); A(l + 1) = t; }
-    int i = l + 1, j = ir;
-    const float a = A(l + 1);
-    for (;;) {
-      do { ++i; } while (A(i) < a);
-      do { --j; } while (A(j) > a);
-      if (j < i) break;
-      t = A(i);
-      A(i) = A(j);
-      A(j) = t;
-    }
-    A(l + 1) = A(j);
-    A(j) = a;
-    if (j >= k) ir = j - 1;
-    if (j <= k) l = i;
+// The wavefront of the calling thread, for prep_selec_wave.
+struct DeviceWave {
+  __device__ __forceinline__ int lane() const { return threadIdx.x & 63; }
+  __device__ __forceinline__ unsigned long long ballot(bool b) const { return __ballot(b); }
+  __device__ __forceinline__ void sync() const {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+    __builtin_amdgcn_wave_barrier();
   }
-}
-
-// The same selection by one wavefront, with the same array afterwards: a partition's scans become
-// two lists of the positions where they stop, ascending from the left (!(A < a)) and descending from
-// the right (!(A > a)), and its exchanges the pairs of list entries that have not crossed.  The
-// scans' last stops are the next entries of their lists, or positions that an exchange has filled
-// if those come first.  ls, rs: n ints each.
-__device__ __forceinline__ void prep_wave_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
-  __builtin_amdgcn_wave_barrier();
-}
-__device__ inline float prep_selec_wave(int k, int n, float* arr, int* ls, int* rs) {
-  const int lane = threadIdx.x & 63;
-  const unsigned long long below = (1ull << lane) - 1;
-  int l = 1, ir = n;
-  float* A = arr - 1;
-  for (;;) {
-    prep_wave_sync();
-    if (ir - l <= 1) {
-      if (ir - 1 == 1) {
-        const float x = A[l], y = A[ir];
-        prep_wave_sync();
-        if (y < x && lane == 0) {
-          A[l] = y;
-          A[ir] = x;
-        }
-        prep_wave_sync();
-      }
-      return A[k];
-    }
-    const int mid = (l + ir) / 2;
-    const float vm = A[mid], v1 = A[l + 1];
-    float x0 = A[l], x1 = vm, x2 = A[ir], t;
-    if (x0 > x2) { t = x0; x0 = x2; x2 = t; }
-    if (x1 > x2) { t = x1; x1 = x2; x2 = t; }
-    if (x0 > x1) { t = x0; x0 = x1; x1 = t; }
-    const float a = x1;
-    prep_wave_sync();
-    if (lane == 0) {
-      A[mid] = v1;
-      A[l] = x0;
-      A[l + 1] = x1;
-      A[ir] = x2;
-    }
-    prep_wave_sync();
-    int nl = 0, nr = 0;
-    for (int b = l + 2; b <= ir; b += 64) {
-      const int p = b + lane;
-      const bool stop = p <= ir && !(A[p <= ir ? p : ir] < a);
-      const unsigned long long m = __ballot(stop);
-      if (stop) ls[nl + __popcll(m & below)] = p;
-      nl += __popcll(m);
-    }
-    for (int b = ir - 1; b > l; b -= 64) {
-      const int p = b - lane;
-      const bool stop = p > l && !(A[p > l ? p : l + 1] > a);
-      const unsigned long long m = __ballot(stop);
-      if (stop) rs[nr + __popcll(m & below)] = p;
-      nr += __popcll(m);
-    }
-    prep_wave_sync();
-    int T = 0;                               // exchanges: entries that have not crossed
-    for (int b = 0; b < min(nl, nr); b += 64) {
-      const int q = b + lane;
-      T += __popcll(__ballot(q < min(nl, nr) && ls[min(q, nl - 1)] <= rs[min(q, nr - 1)]));
-    }
-    for (int b = 0; b < T; b += 64) {
-      const int q = b + lane;
-      if (q < T) {
-        const float x = A[ls[q]], y = A[rs[q]];
-        A[ls[q]] = y;
-        A[rs[q]] = x;
-      }
-    }
-    int i = ls[T], j = rs[T];
-    const int q = T > 0 && ls[T - 1] == rs[T - 1] ? T - 2 : T - 1;
-    if (q >= 0) {
-      i = min(i, rs[q]);
-      j = max(j, ls[q]);
-    }
-    prep_wave_sync();
-    if (lane == 0) {
-      A[l + 1] = A[j];
-      A[j] = a;
-    }
-    if (j >= k) ir = j - 1;
-    if (j <= k) l = i;
-  }
-}
+};
 
 // cosedge_1 (simple_math.f90:1089-1103) and cosedge_inner_1 (:1128-1140), FP32.  sqrtf is the correctly
 // rounded root, which decides the comparisons with the radii; __fsqrt_rn is the bare hardware root.
@@ -522,7 +407,7 @@ __global__ void __launch_bounds__(256) k_prep_mask(float* __restrict__ imgs, int
     int* lists = reinterpret_cast<int*>(edge + 4 * M);
     const int w = tid >> 6, k = M / 2;
     if (w < 2) {
-      const float v = prep_selec_wave(k, M, w ? e1 : e0, lists + 2 * w * M, lists + (2 * w + 1) * M);
+      const float v = prep_selec_wave(DeviceWave{}, k, M, w ? e1 : e0, lists + 2 * w * M, lists + (2 * w + 1) * M);
       if ((tid & 63) == 0) med_s[w] = v;
     }
     __syncthreads();
@@ -534,7 +419,7 @@ __global__ void __launch_bounds__(256) k_prep_mask(float* __restrict__ imgs, int
     }
     __syncthreads();
     if (w < 2) {
-      const float v = prep_selec_wave(k, M, w ? e3 : e2, lists + 2 * w * M, lists + (2 * w + 1) * M);
+      const float v = prep_selec_wave(DeviceWave{}, k, M, w ? e3 : e2, lists + 2 * w * M, lists + (2 * w + 1) * M);
       if ((tid & 63) == 0) med_s[2 + w] = v;
     }
   }

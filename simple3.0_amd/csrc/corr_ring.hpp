@@ -329,10 +329,11 @@ constexpr size_t ring_lds_bytes(int rows) {
 // RST: shifted CC search without shell normalisation whose tiles span at most ring_rows
 // references: the shell's CTF-weighted reference rows are staged once per work-group in LDS and each
 // reference's norm is summed from them (|ref x CTF x shmat|^2 = |ref x CTF|^2), instead of per pair.
-// PRF: pass 1 loads its global operand (per-pair: reference values, RST: shift phases) a shell ahead.
+// PRF (per-pair variant): pass 1 loads its reference values a shell ahead.
 // SPLIT: only the transforms, of the shells of one chunk (RingSplit).
 template <int N, int A, int F, int NT, int W, int RP, bool RST, bool PRF, bool SPLIT>
 __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(W))) k_corr_ring(CorrArgs a, RingSplit sp) {
+  static_assert(!(RST && PRF), "the staged variant loads its shift phases where it uses them");
   using R = RingGeom<N, A>;
   constexpr int B = R::B, H = R::H, S = R::S;
   constexpr int T1 = F * B, TPT1 = (T1 + NT - 1) / NT;
@@ -407,7 +408,7 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(W))) k_
     sqp[c] = 0.f;
     offp[c] = 0.f;
     roff[c] = (RST ? 2u : 16u) * t3;
-    soff[c] = (RST && !PRF ? 2u : 16u) * t3;
+    soff[c] = (RST ? 2u : 16u) * t3;
     slotref[c] = 0;
     if (task < T1 && P < npairs) {
       const int ir = P / a.ns, is = P % a.ns;
@@ -415,7 +416,7 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(W))) k_
       slotref[c] = iref;
       if constexpr (RST) roff[c] += (unsigned int)((ir - rr0) * N);
       else roff[c] += (unsigned int)iref * (unsigned int)(nk * N * 8);
-      soff[c] += (unsigned int)is * (unsigned int)(nk * N * (RST && !PRF ? 1 : 8));
+      soff[c] += (unsigned int)is * (unsigned int)(nk * N * (RST ? 1 : 8));
     }
   }
   float2 acc[TPTL][RP * B];
@@ -497,8 +498,7 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(W))) k_
       for (int c = 0; c < TPT1; ++c)
         if (tid + c * NT < t1)
 #pragma unroll
-          for (int h = 0; h < H; ++h) pre[c][h] = RST ? ld16b(a.shtab + (size_t)kb * N, soff[c], 16 * h * B)
-                                                          : ld16b(refs + (size_t)kb * N, roff[c], 16 * h * B);
+          for (int h = 0; h < H; ++h) pre[c][h] = ld16b(refs + (size_t)kb * N, roff[c], 16 * h * B);
     stage_rows();
   }
   __syncthreads();
@@ -531,9 +531,7 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(W))) k_
         constexpr int T = decltype(tt)::value;
         if constexpr (RST) {
           const float4 r = *reinterpret_cast<const float4*>(rck + roff[c] + 2 * T * B);
-          float4 s;
-          if constexpr (PRF) s = pre[c][T];
-          else s = ld16(a.shtab, soff[c] + (unsigned int)kN + 2 * T * B);
+          const float4 s = ld16(a.shtab, soff[c] + (unsigned int)kN + 2 * T * B);
           const float2 q0 = cmul(make_float2(r.x, r.y), make_float2(s.x, s.y));
           const float2 q1 = cmul(make_float2(r.z, r.w), make_float2(s.z, s.w));
           E[T] = make_float2(q0.x, q1.x);
@@ -558,7 +556,7 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(W))) k_
       if constexpr (PRF)
         static_for<0, H>([&](auto tt) {
           constexpr int T = decltype(tt)::value;
-          pre[c][T] = RST ? ld16b(a.shtab + kX, soff[c], 16 * T * B) : ld16b(refs + kX, roff[c], 16 * T * B);
+          pre[c][T] = ld16b(refs + kX, roff[c], 16 * T * B);
         });
       float e2 = 0.f;
       if constexpr (!RST) {

@@ -55,9 +55,9 @@ struct Fp {
   static constexpr bool fusable = np >= 2 && plan.r[0] == 4 && N % 4 == 0;
 };
 
-// In-place Stockham pass P of F transforms held in LDS (transform f at buf + f S); each thread
+// In-place Stockham pass P of F transforms held in LDS (transform f at buf + f N); each thread
 // stages its butterflies' inputs in registers between two barriers.
-template <int N, int F, int NT, int P, int S = N>
+template <int N, int F, int NT, int P>
 __device__ __forceinline__ void lds_pass(float2* __restrict__ buf, const float2* __restrict__ tw2, int tid) {
   constexpr int R = Fp<N>::R(P);
   constexpr int Ns = Fp<N>::Ns(P);
@@ -72,7 +72,7 @@ __device__ __forceinline__ void lds_pass(float2* __restrict__ buf, const float2*
     if (TASKS % NT == 0 || task < TASKS) {
       const int f = task / nb, j = task % nb;
 #pragma unroll
-      for (int t = 0; t < R; ++t) v[c][t] = buf[f * S + j + t * nb];
+      for (int t = 0; t < R; ++t) v[c][t] = buf[f * N + j + t * nb];
     }
   }
   __syncthreads();
@@ -90,17 +90,17 @@ __device__ __forceinline__ void lds_pass(float2* __restrict__ buf, const float2*
       Dft<R>::run(v[c]);
       const int base = (j / Ns) * Ns * R + jm;
 #pragma unroll
-      for (int t = 0; t < R; ++t) buf[f * S + base + t * Ns] = v[c][t];
+      for (int t = 0; t < R; ++t) buf[f * N + base + t * Ns] = v[c][t];
     }
   }
   __syncthreads();
 }
 
-template <int N, int F, int NT, int P, int PEND, int S = N>
+template <int N, int F, int NT, int P, int PEND>
 __device__ __forceinline__ void lds_passes(float2* buf, const float2* tw2, int tid) {
   if constexpr (P < PEND) {
-    lds_pass<N, F, NT, P, S>(buf, tw2, tid);
-    lds_passes<N, F, NT, P + 1, PEND, S>(buf, tw2, tid);
+    lds_pass<N, F, NT, P>(buf, tw2, tid);
+    lds_passes<N, F, NT, P + 1, PEND>(buf, tw2, tid);
   }
 }
 

@@ -39,7 +39,7 @@ template <int LC, int F>
 __device__ __forceinline__ float2* prep_fft(float2* bufA, float2* bufB, int L, const FftPlan& plan,
                                             const float2* tw2, int tid, int nt) {
   if constexpr (LC > 0) {
-    lds_passes<LC, F, 256, 0, Fp<LC>::np, LC>(bufA, tw2, tid);
+    lds_passes<LC, F, 256, 0, Fp<LC>::np>(bufA, tw2, tid);
     return bufA;
   } else {
     return fft_forward_oop(bufA, bufB, F, L, L, plan, tw2, tid, nt);

@@ -28,7 +28,7 @@ struct RingCfg {
   int F;      // pairs per work-group
   int W;      // wavefronts per SIMD the registers must allow
   int RP;     // rows per last-pass task
-  bool PRF;   // pass 1's global operand loaded a shell ahead
+  bool PRF = false;   // per-pair: reference values loaded a shell ahead
 };
 struct RingRow {
   int n;
@@ -53,7 +53,7 @@ struct Ring {
     if (rst && sp.nsplit > 1)
       hipLaunchKernelGGL((k_corr_ring<N, S.A, S.F, NT, 2, 1, true, false, true>), grid, dim3(NT), lds_r, s, a, sp);
     else if (rst)
-      hipLaunchKernelGGL((k_corr_ring<N, S.A, S.F, NT, S.W, S.RP, true, S.PRF, false>), grid, dim3(NT), lds_r, s, a, sp);
+      hipLaunchKernelGGL((k_corr_ring<N, S.A, S.F, NT, S.W, S.RP, true, false, false>), grid, dim3(NT), lds_r, s, a, sp);
     else if (sp.nsplit > 1)
       hipLaunchKernelGGL((k_corr_ring<N, P.A, P.F, NT, 2, 1, false, false, true>), grid, dim3(NT), lds, s, a, sp);
     else

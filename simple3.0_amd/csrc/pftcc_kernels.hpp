@@ -583,8 +583,8 @@ __device__ __forceinline__ void rot8_step(const Rot8Args a, const Rot8Shell& s, 
 
 // Shells of loads in flight ahead of the arithmetic in k_rot8, and wavefronts per SIMD its registers must
 // allow.  Many items hide their latency by wavefronts (9000 pairs at n 308, 69 shells: 0.52 ms with 1
-// ahead at 7 wavefronts, 0.62 with 4 ahead at 4); few items by loads ahead (shift search of 1000
-// pairs: 10.5 ms with 1 ahead, 10.1 with 4, 10.3 with 6 to 12).  Both take an item's sums in the same order,
+// ahead at 7 wavefronts, 0.62 with 4 ahead at 4); few items by loads ahead (256 at n 308: 48 -> 44
+// us; 6 to 12 ahead no better).  Both take an item's sums in the same order,
 // whatever the items beside it: spreading the shells of a few items over work-groups took one item at
 // n 192 from 16 to 7 us, but a line search that is driven item by item or in batches then saw other bits.
 constexpr int kRot8Ahead = 1, kRot8Waves = 7;

@@ -207,7 +207,7 @@ def test_ring_kernel_keeps_the_generic_kernel_s_accuracy(n, ns, monkeypatch):
 @pytest.mark.parametrize("form", [dict(), dict(match_filt=True), dict(euclid=True)])
 def test_objective_of_an_item_is_the_same_in_every_batch(form):
     """The FP64 objective and gradient of an item have the same bits alone, among a few and among many
-    (the batches of 1024 and 1025 items lie on both sides of k_rot8's variants)."""
+    (1024 and 1025 items of three wavefronts lie on both sides of k_rot8's variants)."""
     say(f"objective in batches: {form}")
     pf, cps = make_case(seed=29, n=192, kfrom=2, kto=40, ctf=True, nrefs=3, nptcls=8, ldim=128, eo_mixed=True, **form)
     lib = to_lib(pf, cps)

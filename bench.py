@@ -31,11 +31,11 @@ METRIC = ("ptcl×ref×rot corr evals/s: plain FP32 vs split-BF16 MFMA @ rel err 
 HBM_PEAK_GBS = 8000.0
 FP32_PEAK_TFLOPS = 157.3
 BF16_PEAK_TFLOPS = 2500.0
-# HBM bytes per launch of k_corr_ring<308,28,17,256,3,2,true,false> at 1000 particles x 200 refs x 169 shifts,
-# from rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE runs of such a search: FETCH 3.076e8 KiB x 2.000 + WRITE
+# HBM bytes per launch of k_corr_ring<308,28,17,256,3,2,true,false,false> at 1000 particles x 200 refs x 169 shifts,
+# from rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE runs of such a search: FETCH 3.152e8 KiB x 2.000 + WRITE
 # 6.216e4 KiB x 1.000, the factors as read from k_copy moving 1 GiB under the same counters
 # (profiles/k_corr_ring_plain_search.md).
-PLAIN_TRAFFIC_BYTES_B1000 = (3.076e8 * 2.0 + 6.216e4) * 1024.0
+PLAIN_TRAFFIC_BYTES_B1000 = (3.152e8 * 2.0 + 6.216e4) * 1024.0
 FP64_PEAK_TFLOPS = 78.6
 
 
@@ -776,7 +776,7 @@ def strategy_form(lib, w, nptcls=10000, reps=2, with_cpu=True):
             "ptcls": n, "refs": w.nrefs, "nrots": nrots, "kinds": res,
             "greedy3d_best_equals_pftcc_search": same,
             "cpu_baseline": cpu,
-            "roofline": {"bound": "valu", "pipe": "VALU fp32", "kernel": "k_corr_ring<308,28,17,256,2,2,false,true>",
+            "roofline": {"bound": "valu", "pipe": "VALU fp32", "kernel": "k_corr_ring<308,28,17,256,2,2,false,true,false>",
                          "achieved": achieved, "peak": FP32_PEAK_TFLOPS, "unit": "TFLOP/s",
                          "frac": achieved / FP32_PEAK_TFLOPS,
                          "note": "unshifted search: one pair per reference, so the staged-reference tile does not apply"}}
@@ -979,7 +979,7 @@ def main():
                      "traffic_note": "HBM bytes per launch from rocprofv3 FETCH_SIZE/WRITE_SIZE, copy-calibrated; "
                                      "compulsory bytes per launch are in hbm_compulsory_bytes",
                      "hbm_compulsory_bytes": bytes_launch,
-                     "kernel": "k_corr_ring<308,28,17,256,3,2,true,false>", "avg_launch_ms": avg_ms, "launches": launches,
+                     "kernel": "k_corr_ring<308,28,17,256,3,2,true,false,false>", "avg_launch_ms": avg_ms, "launches": launches,
                      "flops_per_pair": plain_flops_per_pair(pftsz, w.nk), "pairs_per_launch": pairs_launch,
                      "hbm_compulsory_GBs": bytes_launch / (avg_ms * 1e-3) / 1e9,
                      "hbm_frac": bytes_launch / (avg_ms * 1e-3) / 1e9 / HBM_PEAK_GBS},

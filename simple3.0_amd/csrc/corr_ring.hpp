@@ -19,9 +19,9 @@
 // Bound: VALU issue and the LDS exchange beside it, three wavefronts per SIMD hiding the latency; HBM
 // traffic is small.  Against four to six LDS passes of radix 4 to 11 (radix-4 first, one barrier
 // each) the two register passes take a third of the LDS accesses: 256 particles x 100 references
-// x 49 shifts at n 308, 59 shells: 40.2 -> 32.3 ms; 200 x 1500 at n 400, 79 shells: 24.0 -> 13.5 ms,
-// where the VALU issues in every cycle; against runtime-size passes 200 x 50 x 25 at n 220, 44
-// shells: 26.1 -> 2.8 ms, and 150 x 500 (Euclid) at n 364, 71 shells: 17.3 -> 4.0 ms.
+// x 49 shifts at n 308, 59 shells: 40.2 -> 32.3 ms; 200 x 1500 at n 400, 79 shells: 24.0 -> 13.5 ms
+// (VALU busy 0.89, 1.03 at n 220); against runtime-size passes 200 x 50 x 25 at n 220, 44
+// shells: 26.1 -> 2.9 ms, and 150 x 500 (Euclid) at n 364, 71 shells: 17.3 -> 3.9 ms.
 #pragma once
 #include <type_traits>
 

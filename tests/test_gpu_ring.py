@@ -11,6 +11,7 @@ import pytest
 
 from cases import make_case
 from gpu_helpers import peak_rel_err, say, to_lib
+from pftcc import SRCH_SHC3D
 
 pytestmark = pytest.mark.gpu
 
@@ -246,3 +247,21 @@ def test_pair_is_the_same_in_every_launch(n):
             if ns < 2:
                 assert np.array_equal(lib.gencorrs(3, 11, sh[0] if ns else None), many[10, 2, 0])
         lib.kill()
+
+
+def test_stochastic_walk_does_not_depend_on_the_batch():
+    """A particle's stochastic search ends at the same reference with the same bits among 400 particles and
+    among 7 (few enough that late rounds spread their shells over work-groups)."""
+    say("stochastic walks: n 176, 400 and 7 particles x 90 references")
+    pf, cps = make_case(seed=176, n=176, kfrom=2, kto=30, ctf=True, nrefs=90, nptcls=400, ldim=144, eo_mixed=True)
+    lib = to_lib(pf, cps)
+    rng = np.random.default_rng(9)
+    order = np.stack([rng.permutation(90) + 1 for _ in range(400)])
+    top = lib.gencorrs_batch(np.arange(1, 401)).max(axis=(1, 2, 3))
+    prev = (top * rng.uniform(0.7, 1.0, 400)).astype(np.float32)
+    many = lib.strategy_srch(SRCH_SHC3D, np.arange(1, 401), srch_order=order, prev_corr=prev, ref_corrs=True)
+    sel = np.arange(3, 400, 61)
+    few = lib.strategy_srch(SRCH_SHC3D, sel + 1, srch_order=order[sel], prev_corr=prev[sel], ref_corrs=True)
+    for key in ("best_ref", "best_rot", "best_corr", "nrefs_eval", "found_better", "ref_corrs"):
+        assert np.array_equal(many[key][sel], few[key]), key
+    lib.kill()

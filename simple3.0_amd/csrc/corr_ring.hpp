@@ -675,9 +675,9 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(W))) k_
 // npairs + P) runs the products, sums, inverse transform, normalisation and output of k_corr_ring on the
 // transforms left in sp, in the same order of operations (row A's bins, the mirror of row 0, have
 // sums of their own there and here).  RST: the reference's norm is summed from its rows, as there.
-// Bound: the latency of the loads, so a thread owns MB bins and keeps UB shells of each in flight.  Call of
-// 160 pairs x 47 shells at n 240: 57 us, as with the chunks' sums added by 160 work-groups; 152 us
-// unsplit through the kernels before.
+// Bound: the latency of the loads, so a thread owns MB bins and keeps UB shells of each in flight, and UK
+// shells of the norm's operands (100 pairs, 9 shifts at n 600: 177 us with the norm's loads one by one,
+// 106).  160 pairs x 47 shells at n 240: 56 us per call; 152 us unsplit through the kernels before.
 template <int N, int A, bool RST, int NT>
 __global__ void __launch_bounds__(NT) k_ring_finish(CorrArgs a, RingSplit sp, int npairs) {
   using R = RingGeom<N, A>;
@@ -700,29 +700,48 @@ __global__ void __launch_bounds__(NT) k_ring_finish(CorrArgs a, RingSplit sp, in
     const int ir = P / a.ns, iref = a.rlist ? a.rlist[ir] : ir;
     const float2* ref = (a.iseven[ip] ? a.refs_even : a.refs_odd) + (size_t)iref * nk * N;
     const float* ctf = a.ctf ? a.ctf + (size_t)ip * nk * N : nullptr;
+    constexpr int UK = 16 / JP;
     double s = 0.0;
-#pragma unroll 8
-    for (int kk = 0; kk < kloop; ++kk)
+    for (int k0 = 0; k0 < kloop; k0 += UK) {
+      float2 r[UK][JP];
+      float cv[UK][JP];
 #pragma unroll
-      for (int u = 0; u < JP; ++u) {
-        const int j = tid + u * NT;
-        if (N % NT == 0 || j < N) {
-          const float cv = ctf ? ctf[kk * N + j] : 1.0f;
-          const float2 r = ref[kk * N + j], q = make_float2(r.x * cv, r.y * cv);
-          s += (double)fmaf(q.y, q.y, q.x * q.x);
+      for (int v = 0; v < UK; ++v)
+#pragma unroll
+        for (int u = 0; u < JP; ++u) {
+          const int e = min(k0 + v, kloop - 1) * N + min(tid + u * NT, N - 1);
+          r[v][u] = ref[e];
+          cv[v][u] = ctf ? ctf[e] : 1.0f;
         }
-      }
+#pragma unroll
+      for (int v = 0; v < UK; ++v)
+#pragma unroll
+        for (int u = 0; u < JP; ++u)
+          if (k0 + v < kloop && (N % NT == 0 || tid + u * NT < N)) {
+            const float2 q = make_float2(r[v][u].x * cv[v][u], r[v][u].y * cv[v][u]);
+            s += (double)fmaf(q.y, q.y, q.x * q.x);
+          }
+    }
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
     if (lane == 0) rsq[tid >> 6] = s;
   } else if (tid < B) {
     const float* e = sp.es + (size_t)pair * kloop * B + tid;
+    constexpr int UK = 16;
     float s = 0.f, o = 0.f;
-#pragma unroll 8
-    for (int kk = 0; kk < kloop; ++kk) {
-      const float e2 = e[kk * B];
-      if (kk < a.knorm) s += e2;
-      if (a.mode == 1 && kk < kc) o = fmaf(a.shellw[(size_t)ip * nk + kk], e2, o);
+    for (int k0 = 0; k0 < kloop; k0 += UK) {
+      float e2[UK], wk[UK];
+#pragma unroll
+      for (int v = 0; v < UK; ++v) {
+        const int k = min(k0 + v, kloop - 1);
+        e2[v] = e[k * B];
+        wk[v] = a.mode == 1 ? a.shellw[(size_t)ip * nk + min(k, kc - 1)] : 0.f;
+      }
+#pragma unroll
+      for (int v = 0; v < UK; ++v) {
+        if (k0 + v < a.knorm) s += e2[v];
+        if (k0 + v < kc) o = fmaf(wk[v], e2[v], o);
+      }
     }
     sqs[tid] = s;
     offs[tid] = o;

@@ -385,7 +385,7 @@ __device__ __forceinline__ float prep_cosedge_inner(float x, float y, float widt
 // M x M image per work-group.  LDS: the four edges and two wavefronts' lists.  The first two edges are
 // independent, and so are the other two, whose corners are as the first two calls left them.
 // Bound: the chain of partitions (a selection is about 8 of them) and one read and write of the
-// image: 1000 images of box 128 157 us with the four selections in one thread, 63 us.
+// image: 1000 images of box 128 157 us with the four selections in one thread, 65 us.
 __global__ void __launch_bounds__(256) k_prep_mask(float* __restrict__ imgs, int M, float mskrad, float inner,
                                                    float width, int minlen, const float* __restrict__ instr_w) {
   extern __shared__ float edge[];            // [4][M], lists [4][M]
